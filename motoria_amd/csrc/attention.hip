@@ -673,28 +673,25 @@ __global__ __launch_bounds__(256) void k_attn_mix_b(float *__restrict__ scores, 
 // 0 .. group - 1 of wavefront 0, one head each. Mix: thread (element
 // tid % AG_HD, heads tid / AG_HD + 2 j), the value rows read 16 positions
 // ahead of their additions. Scores (row stride sld, a multiple of 4) in
-// LDS behind the key rows (SC_LDS) or at scores + ((t * nh + h) * sld).
+// LDS behind the key rows: below AB_MIN_CTX positions they always fit.
 constexpr int AG_HD = 128, AG_KLD = AG_HD + 4, AG_MAXG = 16;
 constexpr size_t AG_LDS_MAX = 150 * 1024;
-size_t ag_lds(int group, int sld, bool sc_lds) {
-    return (size_t)(256 / group) * AG_KLD * 4 + (sc_lds ? (size_t)group * sld * 4 : 0);
+size_t ag_lds(int group, int sld) {
+    return (size_t)(256 / group) * AG_KLD * 4 + (size_t)group * sld * 4;
 }
 
-template <bool SC_LDS>
 __global__ __launch_bounds__(256) void k_attn_group_b(const float *__restrict__ q,
                                                       const float *__restrict__ kc,
                                                       const float *__restrict__ vc, int pos,
                                                       int nh, int group, int kvd, float scale,
-                                                      float *__restrict__ scores, int sld,
-                                                      float *__restrict__ att) {
+                                                      int sld, float *__restrict__ att) {
     extern __shared__ __align__(16) float ag_sh[];
     __shared__ uint64_t etab[32];
     __shared__ float sum_sh[AG_MAXG];
     const int g = blockIdx.x, t = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
     const int wave = tid >> 6, np = pos + t + 1, C = 256 / group;
     float *kt = ag_sh;
-    float *sc = SC_LDS ? ag_sh + (size_t)C * AG_KLD
-                       : scores + ((size_t)t * nh + (size_t)g * group) * sld;
+    float *sc = ag_sh + (size_t)C * AG_KLD;
     if (tid < 32) etab[tid] = mia_expf_tab[tid];
     {
         const int hh = tid / C, c = tid % C;
@@ -808,6 +805,21 @@ __global__ __launch_bounds__(256) void k_attn_group_b(const float *__restrict__ 
     }
 }
 
+// Batches whose scores and mix run in tiles (attn_batch.hip) rather than a
+// workgroup per (key/value head, token), whose time is that of one token's
+// chain while the chip has room: long contexts, where a group's scores fill
+// a CU's LDS, and many tokens. Measured at 32/4 heads (a layer's whole call,
+// us, workgroup per token / tiles): 8 tokens at 600 162/164, at 1000 209/208,
+// at 2000 353/315; 100 at 600 207/208, at 1000 259/255, at 2000 601/381; at
+// position 0 200 tokens 209/209, 300 277/270, 500 435/406.
+constexpr int AB_MIN_CTX = 1000, AB_MIN_N = 250;
+static_assert((256 * AG_KLD + AB_MIN_CTX) * 4 <= AG_LDS_MAX &&
+                  (256 / AG_MAXG * AG_KLD + AG_MAXG * AB_MIN_CTX) * 4 <= AG_LDS_MAX,
+              "k_attn_group_b's scores fit LDS at every group");
+bool tiles_fit(const mhip_attn_dims *s, int n, int end) {
+    return s->head_dim == AG_HD && (end >= AB_MIN_CTX || n >= AB_MIN_N);
+}
+
 constexpr size_t HEAD_LDS_MAX = 150 * 1024;  // dynamic LDS of k_attn_head
 size_t head_lds(int hd, int max_seq) { return ((size_t)4 * hd + (size_t)max_seq) * sizeof(float); }
 
@@ -918,9 +930,15 @@ int mhip_attention(mhip_ctx *c, const mhip_attn_dims *s, const float *d_attn_nor
     return mhip::check_launch(c, "attention");
 }
 
-// Tokens per pass of the scores kept in device memory (contexts too long for
-// LDS, other head shapes): the scratch holds this many tokens' scores.
+// Tokens per pass of k_attn_scores_b: the scratch holds this many tokens'
+// scores (or a pass of the tiles').
 constexpr int AB_SUB = 64;
+
+static size_t scores_bytes(const mhip_attn_dims *s, int n, int max_seq) {
+    const size_t sub = (size_t)(n < AB_SUB ? n : AB_SUB) * s->n_heads * (size_t)((max_seq + 3) & ~3) * 4;
+    const size_t tiles = tiles_fit(s, n, max_seq) ? mhip::attn_batch_scratch(s->n_heads, n, max_seq) : 0;
+    return sub > tiles ? sub : tiles;
+}
 
 size_t mhip_attention_batch_scratch_bytes(const mhip_attn_dims *s, int n, int max_seq) {
     if (!s || n <= 0 || max_seq <= 0) return 0;
@@ -929,9 +947,7 @@ size_t mhip_attention_batch_scratch_bytes(const mhip_attn_dims *s, int n, int ma
     return align256(N * d * 4) + align256(N * d) + align256(N * (d / QK) * 4) +
            align256(N * qd * 4) + 2 * align256(N * kvd * 4) + align256(N * qd * 4) +
            align256(N * qd) + align256(N * (qd / QK) * 4) + align256(N * d * 2) +
-           align256(N * qd * 2) +
-           align256((size_t)(n < AB_SUB ? n : AB_SUB) * s->n_heads * (size_t)((max_seq + 3) & ~3) * 4) +
-           align256(16);
+           align256(N * qd * 2) + align256(scores_bytes(s, n, max_seq)) + align256(16);
 }
 
 }  // extern "C"
@@ -1051,16 +1067,13 @@ int mhip_attention_batch(mhip_ctx *c, const mhip_attn_dims *s, const float *d_at
     _Float16 *xh = (_Float16 *)take(N * d * 2);
     _Float16 *atth = (_Float16 *)take(N * qd * 2);
     const int sld = (max_seq + 3) & ~3;  // row stride of the scores
-    float *scores = (float *)take((size_t)(n < AB_SUB ? n : AB_SUB) * nh * (size_t)sld * 4);
+    const size_t sbytes = scores_bytes(s, n, max_seq);
+    float *scores = (float *)take(sbytes);
     int *status = (int *)take(16);
     hipStream_t st = c->stream;
     static int lds_set[64];  // per device ordinal
     if (c->device >= 0 && c->device < 64 && !lds_set[c->device]) {
-        if (mhip::check(c, hipFuncSetAttribute((const void *)k_attn_group_b<true>,
-                                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               (int)AG_LDS_MAX),
-                        "attention LDS attribute") ||
-            mhip::check(c, hipFuncSetAttribute((const void *)k_attn_group_b<false>,
+        if (mhip::check(c, hipFuncSetAttribute((const void *)k_attn_group_b,
                                                hipFuncAttributeMaxDynamicSharedMemorySize,
                                                (int)AG_LDS_MAX),
                         "attention LDS attribute"))
@@ -1090,19 +1103,16 @@ int mhip_attention_batch(mhip_ctx *c, const mhip_attn_dims *s, const float *d_at
         q, k, v, d_q_norm, d_k_norm, d_rope, pos, nh, nkv, hd, s->norm_eps, d_kc, d_vc);
     const float scale = 1.0f / sqrtf((float)hd);
     const int group = nh / nkv;
-    if (hd == AG_HD && group <= AG_MAXG && 256 % group == 0) {
-        // the group's heads together; their scores in LDS while they fit
+    const bool tiles = tiles_fit(s, n, pos + n);
+    if (tiles) {
+        // scores, softmax, mix and Q8 of the rows (fp16 codes for the matrix cores)
+        mhip::launch_attn_batch(st, q, d_kc, d_vc, pos, n, nh, nkv, scale, scores, sbytes,
+                                mm ? nullptr : attq, mm ? atth : nullptr, atts);
+    } else if (hd == AG_HD && group <= AG_MAXG && 256 % group == 0) {
+        // the group's heads together, their scores in LDS
         const int sl = (pos + n + 3) & ~3;
-        if (ag_lds(group, sl, true) <= AG_LDS_MAX)
-            k_attn_group_b<true><<<dim3(nkv, n), 256, ag_lds(group, sl, true), st>>>(
-                q, d_kc, d_vc, pos, nh, group, kvd, scale, nullptr, sl, att);
-        else
-            for (int t0 = 0; t0 < n; t0 += AB_SUB) {
-                const int ns = n - t0 < AB_SUB ? n - t0 : AB_SUB;
-                k_attn_group_b<false><<<dim3(nkv, ns), 256, ag_lds(group, sld, false), st>>>(
-                    q + (size_t)t0 * qd, d_kc, d_vc, pos + t0, nh, group, kvd, scale, scores, sld,
-                    att + (size_t)t0 * qd);
-            }
+        k_attn_group_b<<<dim3(nkv, n), 256, ag_lds(group, sl), st>>>(q, d_kc, d_vc, pos, nh, group,
+                                                                     kvd, scale, sl, att);
     } else {
         for (int t0 = 0; t0 < n; t0 += AB_SUB) {
             const int ns = n - t0 < AB_SUB ? n - t0 : AB_SUB;
@@ -1114,10 +1124,11 @@ int mhip_attention_batch(mhip_ctx *c, const mhip_attn_dims *s, const float *d_at
         }
     }
     if (mhip::check_launch(c, "attention batch scores")) return -1;
-    k_quant_rows<<<mhip::blocks_for(N * qd / QK, 256), 256, 0, st>>>(att, (int)(N * qd / QK),
-                                                                      attq, atts);
+    if (!tiles)
+        k_quant_rows<<<mhip::blocks_for(N * qd / QK, 256), 256, 0, st>>>(att, (int)(N * qd / QK),
+                                                                          attq, atts);
     if (mm) {
-        k_codes_h<<<mhip::blocks_for(N * qd, 256), 256, 0, st>>>(attq, N * qd, atth);
+        if (!tiles) k_codes_h<<<mhip::blocks_for(N * qd, 256), 256, 0, st>>>(attq, N * qd, atth);
         float *outs[1] = {d_x};
         const int r0[4] = {0, d, d, d};
         rows_mfma(st, pk, 3, 1, outs, r0, qd / QK, n, atth, atts, d_x, d);

@@ -60,6 +60,14 @@ int decode_noalloc_setup(mhip_ctx *c);
 void launch_rmsnorm_q8(hipStream_t st, const float *x, const float *w, float *xn, int8_t *xq,
                        float *xs, int T, int d, float eps, int force_seq, int *status);
 
+// Scores, softmax, mix and Q8 of a prompt batch, head_dim 128 (attn_batch.hip):
+// codes to attq, or as fp16 integers to atth; `bytes` of scratch as
+// attn_batch_scratch gives for (at least) these tokens and positions.
+size_t attn_batch_scratch(int nh, int n, int max_seq);
+void launch_attn_batch(hipStream_t st, const float *q, const float *kc, const float *vc, int pos,
+                       int n, int nh, int nkv, float scale, void *scratch, size_t bytes,
+                       int8_t *attq, _Float16 *atth, float *atts);
+
 // Matrix-core expert products (moe_gemm.hip).
 bool gemm_path_fits(const mhip_dims *s);
 int gemm_max_tiles(int A, int E);
