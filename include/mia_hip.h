@@ -313,12 +313,11 @@ int mhip_attention_batch(mhip_ctx *c, const mhip_attn_dims *s, const float *d_at
                          const void *d_pack, void *d_scratch, int flags);
 /* The layer's Q, K, V and O weights repacked for mhip_attention_batch's
  * matrix-core rows (no counterpart in the reference): codes as fp16
- * integers, scales block-major; d_pack holds mhip_attention_pack_bytes(s)
+ * integers in the matrix instruction's order, scales block-major; d_pack holds mhip_attention_pack_bytes(s)
  * bytes (0 for shapes whose rows are not multiples of 64, which keep the
- * vector kernels). With d_pack given, batches of 512
- * tokens or more form their Q/K/V and O rows on the matrix cores, with the
- * same bits (exact block dots, block terms in block order); NULL keeps the
- * vector kernels. */
+ * vector kernels). With d_pack given, the batch's
+ * Q/K/V and O rows form on the matrix cores, with the same bits (exact block
+ * dots, block terms in block order); NULL keeps the vector kernels. */
 size_t mhip_attention_pack_bytes(const mhip_attn_dims *s);
 int mhip_attention_pack(mhip_ctx *c, const mhip_attn_dims *s, const void *d_wq, const void *d_wk,
                         const void *d_wv, const void *d_wo, void *d_pack);

@@ -270,8 +270,9 @@ __global__ __launch_bounds__(320) void k_ab_stat(const float *__restrict__ S, in
 // (blocks of 16 x 16): the rows' probabilities (the exponential again, over
 // the sum) and the value rows staged in LDS XU positions at a time, the next
 // ones requested ahead; then Q8 of each row's 32 values (a wavefront's 32
-// elements are one block, quant.c:11-27): codes as int8 (attq) or as fp16
-// integers (atth) and scales [t][nh * 4]. A position that only some rows of
+// elements are one block, quant.c:11-27): codes as int8 (attq) and scales
+// [t][nh * 4], or (atth) as the row kernels read them: fp16 integers in
+// fragments of 16 tokens from token tb on, scales [nh * 4][ld]. A position that only some rows of
 // the tile read (the batch's own tokens) is added to those alone.
 constexpr int XR = 32, XU = 32, XLD = XU + 4;
 
@@ -281,7 +282,7 @@ __global__ __launch_bounds__(256, 4) void k_ab_mix(const float *__restrict__ S, 
                                                    int n, int nh, int group, int kvd,
                                                    int8_t *__restrict__ attq,
                                                    _Float16 *__restrict__ atth,
-                                                   float *__restrict__ atts) {
+                                                   float *__restrict__ atts, int tb, int ld) {
     __shared__ __align__(16) float ps[XR * XLD], vs[XU * HD];
     __shared__ uint64_t etab[32];
     int g, rt;
@@ -369,16 +370,21 @@ __global__ __launch_bounds__(256, 4) void k_ab_mix(const float *__restrict__ S, 
             const float qi = d != 0.0f ? 1.0f / d : 0.0f;
             if (row >= rows) continue;
             const int t = row / group, h = g * group + (row - t * group);
-            const size_t o = ((size_t)t * nh + h) * HD + 32 * wave + c16;
             const int8_t q0 = (int8_t)roundf(o0 * qi), q1 = (int8_t)roundf(o1 * qi);
+            const int ob = h * (HD / 32) + wave;  // the block of the output row
             if (atth) {
-                atth[o] = (_Float16)q0;
-                atth[o + 16] = (_Float16)q1;
+                // codes 8 c .. + 7 of token t at lane 16 c + t % 16
+                _Float16 *f = atth + ((size_t)((tb + t) / 16) * (nh * (HD / 32)) + ob) * 512 +
+                              (c16 / 8) * 128 + ((tb + t) % 16) * 8 + c16 % 8;
+                f[0] = (_Float16)q0;
+                f[256] = (_Float16)q1;
+                if (c16 == 0) atts[(size_t)ob * ld + tb + t] = d;
             } else {
+                const size_t o = ((size_t)(tb + t) * nh + h) * HD + 32 * wave + c16;
                 attq[o] = q0;
                 attq[o + 16] = q1;
+                if (c16 == 0) atts[(size_t)(tb + t) * nh * (HD / 32) + ob] = d;
             }
-            if (c16 == 0) atts[((size_t)t * nh + h) * (HD / 32) + wave] = d;
         }
 }
 
@@ -404,7 +410,7 @@ size_t attn_batch_scratch(int nh, int n, int max_seq) {
 
 void launch_attn_batch(hipStream_t st, const float *q, const float *kc, const float *vc, int pos,
                        int n, int nh, int nkv, float scale, void *scratch, size_t bytes,
-                       int8_t *attq, _Float16 *atth, float *atts) {
+                       int8_t *attq, _Float16 *atth, float *atts, int ld) {
     const int group = nh / nkv, kvd = nkv * HD, qd = nh * HD;
     const int sld = (pos + n + 3) & ~3, pld = part_ld(sld);
     const size_t fit = (bytes - 3 * 256) / token_bytes(nh, sld);
@@ -420,9 +426,7 @@ void launch_attn_batch(hipStream_t st, const float *q, const float *kc, const fl
         k_ab_stat<<<blocks_for((size_t)ns * nh, MR), 320, 0, st>>>(S, sld, pmax, pld, p0, ns * nh,
                                                                    nh, stat);
         k_ab_mix<<<(unsigned)tx.blocks(), 256, 0, st>>>(
-            S, sld, stat, vc, tx, p0, ns, nh, group, kvd,
-            attq ? attq + (size_t)t0 * qd : nullptr, atth ? atth + (size_t)t0 * qd : nullptr,
-            atts + (size_t)t0 * (qd / 32));
+            S, sld, stat, vc, tx, p0, ns, nh, group, kvd, attq, atth, atts, t0, ld);
     }
 }
 

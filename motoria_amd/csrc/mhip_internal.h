@@ -61,12 +61,26 @@ void launch_rmsnorm_q8(hipStream_t st, const float *x, const float *w, float *xn
                        float *xs, int T, int d, float eps, int force_seq, int *status);
 
 // Scores, softmax, mix and Q8 of a prompt batch, head_dim 128 (attn_batch.hip):
-// codes to attq, or as fp16 integers to atth; `bytes` of scratch as
-// attn_batch_scratch gives for (at least) these tokens and positions.
+// codes to attq and scales [t][nh * 4] to atts, or (atth) the row kernels'
+// token fragments and block-major scales [nh * 4][ld]; `bytes` of scratch
+// as attn_batch_scratch gives for (at least) these tokens and positions.
 size_t attn_batch_scratch(int nh, int n, int max_seq);
 void launch_attn_batch(hipStream_t st, const float *q, const float *kc, const float *vc, int pos,
                        int n, int nh, int nkv, float scale, void *scratch, size_t bytes,
-                       int8_t *attq, _Float16 *atth, float *atts);
+                       int8_t *attq, _Float16 *atth, float *atts, int ld);
+
+// The weight rows of a prompt batch on the matrix cores (attn_rows.hip):
+// weights packed by rows_pack (shapes rows_pack_fits), tokens as fragments of
+// 16 and block-major scales of stride ld, both allocated to a multiple of 128
+// tokens (what lies past token n - 1 is read, its results are not stored).
+bool rows_pack_fits(const mhip_attn_dims *s);
+void rows_pack(hipStream_t st, const mhip_attn_dims *s, const void *const *w, void *pack);
+void rows_token_frags(hipStream_t st, const int8_t *q, const float *s, int n, int nb, int ld,
+                      _Float16 *o, float *os);
+void rows_qkv(hipStream_t st, const mhip_attn_dims *s, const void *pack, int n, const _Float16 *xh,
+              const float *xs, int ld, float *q, float *k, float *v);
+void rows_o(hipStream_t st, const mhip_attn_dims *s, const void *pack, int n, const _Float16 *xh,
+            const float *xs, int ld, float *x);
 
 // Matrix-core expert products (moe_gemm.hip).
 bool gemm_path_fits(const mhip_dims *s);

@@ -43,14 +43,12 @@ class Layer:
         self.kn = up(rng.uniform(0.5, 2.5, HD).astype(np.float32))
         ang = rng.uniform(0, 6.28, (max_seq, HD // 2))
         self.rope = up(np.stack([np.cos(ang), np.sin(ang)], -1))
-        self.pack = None
-        nb = self.L.mhip_attention_pack_bytes(ctypes.byref(self.a))
-        if nb:
-            self.pack = torch.empty(nb, dtype=torch.uint8, device="cuda")
-            torch.cuda.synchronize()
-            self.g.check(self.L.mhip_attention_pack(self.g.h, ctypes.byref(self.a),
-                                                    *[t.data_ptr() for t in self.w],
-                                                    self.pack.data_ptr()), "pack")
+        self.pack = torch.empty(self.L.mhip_attention_pack_bytes(ctypes.byref(self.a)),
+                                dtype=torch.uint8, device="cuda")
+        torch.cuda.synchronize()
+        self.g.check(self.L.mhip_attention_pack(self.g.h, ctypes.byref(self.a),
+                                                *[t.data_ptr() for t in self.w],
+                                                self.pack.data_ptr()), "pack")
 
     def close(self):
         self.g.close()
@@ -66,7 +64,7 @@ class Layer:
                 [self.qn.data_ptr(), self.kn.data_ptr(), self.rope.data_ptr(), kc.data_ptr(),
                  vc.data_ptr()])
 
-    def batch(self, x, kc, vc, pos):
+    def batch(self, x, kc, vc, pos, packed=True, flags=0):
         t, n = self.torch, x.shape[0]
         nb = self.L.mhip_attention_batch_scratch_bytes(ctypes.byref(self.a), n, self.max_seq)
         scratch = t.full((nb,), 255, dtype=t.uint8, device="cuda")
@@ -74,7 +72,7 @@ class Layer:
         t.cuda.synchronize()
         self.g.check(self.L.mhip_attention_batch(
             self.g.h, ctypes.byref(self.a), *self.args(kc, vc), pos, n, self.max_seq, out.data_ptr(),
-            self.pack.data_ptr() if self.pack is not None else None, scratch.data_ptr(), 0), "batch")
+            self.pack.data_ptr() if packed else None, scratch.data_ptr(), flags), "batch")
         t.cuda.synchronize()
         return out
 
@@ -106,31 +104,36 @@ def test_batch_equals_tokens(n, pos, nh, nkv):
         kc, vc = lay.cache(pos)
         k2, v2 = kc.clone(), vc.clone()
         x = lay.up(lay.rng.standard_normal((n, 256)).astype(np.float32))
-        got = lay.batch(x, kc, vc, pos)
+        got = lay.batch(x, kc.clone(), vc.clone(), pos, packed=False)
         want = torch.cat([lay.token(x[i:i + 1], k2, v2, pos + i) for i in range(n)])
         assert torch.isfinite(want).all()
-        assert np.array_equal(bits(got), bits(want))
+        assert np.array_equal(bits(got), bits(want)), "vector rows"
+        got = lay.batch(x, kc, vc, pos, flags=M.MHIP_FORCE_SEQ_RMS if n % 2 else 0)
+        assert np.array_equal(bits(got), bits(want)), "matrix-core rows"
         assert np.array_equal(bits(kc[:pos + n]), bits(k2[:pos + n]))
         assert np.array_equal(bits(vc[:pos + n]), bits(v2[:pos + n]))
     finally:
         lay.close()
 
 
-@pytest.mark.parametrize("n", [511, 512, 600])
+@pytest.mark.parametrize("n", [1, 15, 33, 64, 100, 511, 512, 577])
 def test_batch_rows_on_matrix_cores(n):
-    """Around the size from which the weight rows take the matrix cores."""
+    """The weight rows on the matrix cores, 32 (from 512 tokens 64) tokens to
+    a workgroup in fragments of 16: dimensions of one and of several 64-row
+    tiles, more blocks and fewer than the ring has stages."""
     torch = pytest.importorskip("torch")
     say("test_batch_rows_on_matrix_cores n=%d" % n)
-    lay = Layer(torch, 256, 8, 2, n + 9, n)
-    try:
-        kc, vc = lay.cache(9)
-        k2, v2 = kc.clone(), vc.clone()
-        x = lay.up(lay.rng.standard_normal((n, 256)).astype(np.float32))
-        got = lay.batch(x, kc, vc, 9)
-        want = torch.cat([lay.token(x[i:i + 1], k2, v2, 9 + i) for i in range(n)])
-        assert np.array_equal(bits(got), bits(want))
-    finally:
-        lay.close()
+    for dim, nh, nkv in ((64, 2, 1), (320, 8, 2)):
+        lay = Layer(torch, dim, nh, nkv, n + 9, n)
+        try:
+            kc, vc = lay.cache(9)
+            k2, v2 = kc.clone(), vc.clone()
+            x = lay.up(lay.rng.standard_normal((n, dim)).astype(np.float32))
+            got = lay.batch(x, kc, vc, 9)
+            want = torch.cat([lay.token(x[i:i + 1], k2, v2, 9 + i) for i in range(n)])
+            assert np.array_equal(bits(got), bits(want))
+        finally:
+            lay.close()
 
 
 def test_batch_in_passes():
