@@ -58,6 +58,11 @@ __device__ __forceinline__ void dma16(unsigned lds, const void *g) {
     asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(g)
                  : "memory", "m0");
 }
+// The same with 4 bytes per lane.
+__device__ __forceinline__ void dma4(unsigned lds, const void *g) {
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(g)
+                 : "memory", "m0");
+}
 #pragma clang diagnostic pop
 
 // A DPP move of x (lanes of rows outside ROWS keep their own value, resp. 0

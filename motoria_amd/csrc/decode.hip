@@ -63,6 +63,7 @@
 // src/model/forward.c:118-165) before that layer's MoE, so a whole decode
 // token is one launch (forward.c:210-213).
 #include <mutex>
+#include <type_traits>
 
 #include "attn_common.h"
 #include "mhip_internal.h"
@@ -137,6 +138,8 @@ struct AttnXWs {
     alignas(256) tw atts[at::NBO];     // their block scales
     alignas(256) tw xa[D];             // x after the attention
     alignas(256) tw xl[NX][D];         // the same, republished in each XCD's L2
+    // long contexts: the scores of each XCD's four query heads
+    alignas(256) tw sc[NX][at::NH / NX][MHIP_MODEL_STACK_MAX_SEQ];
 };
 
 struct DecodeArgs {
@@ -571,9 +574,268 @@ template <class T> __device__ __forceinline__ T *uniform_ptr(T *p) {
     return (T *)(((uint64_t)hi << 32) | lo);
 }
 
+// ---- the heads of a long context, over a whole XCD -----------------------------------
+//
+// From LONG_MIN_POS on a head's work (scores, softmax, mix over pos + 1
+// positions) is spread over its XCD: XCD x holds query heads 4 x .. 4 x + 3,
+// all of key/value group x / 2. Each of its 32 workgroups scores a 32nd of
+// the positions for the four heads (its key rows copied into LDS while the
+// q/k/v rows form) and publishes the scores in the XCD's L2; workgroups of
+// rank < 16 then take a head and 32 of its elements each: softmax, and the
+// position-ordered mix as a pipeline: wavefronts 1-7 form the products
+// p_t v_t of LC positions in an LDS ring, from which wavefront 0 adds the
+// previous LC's, four to a read, so that the chain of one addition per
+// position (~5 cycles) is all that is serial. Every value and its order are
+// head_run's.
+constexpr int LH = at::NH / NX;        // query heads of an XCD
+constexpr int LKR = 80;                // key rows a workgroup stages at a time
+constexpr int LQ = at::HD + 4;         // q row stride
+constexpr int LU = 3;                  // four-position slots of a producer's half wavefront
+constexpr int LSLOT = (NWAVE - 1) * 2 * LU, LC = 4 * LSLOT;  // slots, positions of a ring buffer
+constexpr int LEL = 32, LQT = at::HD / LEL;  // elements of a mixing workgroup, such parts of a head
+static_assert(LH * LQT <= WPX && LH == 4 && at::GROUP == 2 * LH, "a head's four parts on its XCD");
+static_assert(LKR * LH <= NT, "a score per thread");
+struct LongLds {
+    alignas(16) float tq[LH][LQ], qs[LH][LQ];
+    alignas(16) float tk[at::HD], ks[at::HD], tv[at::HD];
+    union alignas(16) {
+        float k[LKR][at::KLD];              // staged key rows
+        float4 ring[2][LSLOT][LEL];          // products of four positions of an element
+    };
+    float touch[64];                        // (target of the value rows' requests)
+    float red[NWAVE], inv[LH + 1], sum;
+    alignas(16) int8_t hq[LEL];
+};
+
+// This workgroup's key rows p .. p + m - 1 of its positions t0 .. into LDS.
+__device__ __forceinline__ void long_stage_keys(LongLds &s, at::gptr<const float> kg, int t0, int m,
+                                                int lane, int wave) {
+    const int half = lane >> 5, c = lane & 31;
+    const unsigned ks = (unsigned)(uintptr_t)&s.k[0][0];
+    for (int q = wave; 2 * q < m; q += NWAVE) {
+        const int r = min(2 * q + half, m - 1);
+        const float *src = (const float *)(kg + (size_t)(t0 + r) * at::KVD + 4 * c);
+        const unsigned k0 = __builtin_amdgcn_readfirstlane(ks + (unsigned)(2 * q * at::KLD * 4));
+        const unsigned k1 = __builtin_amdgcn_readfirstlane(k0 + (unsigned)(at::KLD * 4 - 32 * 16));
+        if (half == 0) at::dma16(k0, src);
+        else if (2 * q + 1 < m) at::dma16(k1, src);
+    }
+}
+
+struct LongPre : at::HeadRope {
+    int t0, cnt;  // this workgroup's positions
+};
+__device__ __forceinline__ void long_prefetch(LongPre &p, LongLds &s, int rank, int pos,
+                                              at::gptr<const float> kg, at::gptr<const float> vg,
+                                              at::gptr<const float> q_norm,
+                                              at::gptr<const float> k_norm,
+                                              at::gptr<const double> rope, int tid, int lane,
+                                              int wave) {
+    const int n = pos + 1, c = (n + WPX - 1) / WPX;
+    p.t0 = min(rank * c, n);
+    p.cnt = min(c, n - p.t0);
+    if (tid < (LH + 1) * 64) {
+        const at::gptr<const float> w = tid < LH * 64 ? q_norm : k_norm;
+        const at::gptr<const double> rp = rope + (size_t)pos * at::HD;
+        p.rw0 = w[lane];
+        p.rw1 = w[lane + at::HD / 2];
+        p.rc = rp[2 * lane];
+        p.rs = rp[2 * lane + 1];
+    }
+    long_stage_keys(s, kg, p.t0, min(p.cnt, LKR), lane, wave);
+    // its value rows requested into the XCD's L2, a word of each 128 bytes
+    const unsigned dst = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)&s.touch[0]);
+    for (int i = tid; i < p.cnt * 4; i += NT)
+        at::dma4(dst, (const float *)(vg + (size_t)(p.t0 + i / 4) * at::KVD + (i % 4) * 32));
+}
+
+// The part of the heads that every workgroup does: q (and the new k) normed
+// and rotated, the cache rows appended, this workgroup's scores published.
+__device__ __forceinline__ void long_scores(const DecodeArgs &a, LongLds &s, DecodeWs *ws,
+                                            const LongPre &p, at::gptr<float> kg,
+                                            at::gptr<float> vg, int xcd, int rank, int tid, int lane,
+                                            int wave, unsigned tag) {
+    const int g = xcd / 2, pos = a.pos;
+    AttnXWs *xw = a.xw;
+    {
+        // q of the four heads (a word per thread), then k and v of the group
+        float v[2];
+        if (tid < 2 * at::HD) {
+            const int kv = at::QD + (tid < at::HD ? 0 : at::KVD - at::HD) + g * at::HD + tid;
+            get_tagged<2, false>(ws, &xw->qkv[LH * at::HD * xcd + tid],
+                                 kv - (LH * at::HD * xcd + tid), tag, v);
+            if (tid < at::HD) s.tk[tid] = v[1];
+            else s.tv[tid - at::HD] = v[1];
+        } else {
+            get_tagged<1, false>(ws, &xw->qkv[LH * at::HD * xcd + tid], 0, tag, v);
+        }
+        s.tq[tid / at::HD][tid % at::HD] = v[0];
+    }
+    __builtin_amdgcn_s_waitcnt(at::WAIT_VM0);  // this wavefront's key rows are in
+    __syncthreads();
+    if (wave <= LH) {
+        const float inv = at::head_inv_wave(wave < LH ? s.tq[wave] : s.tk, a.eps, lane,
+                                            (a.flags & MHIP_FORCE_SEQ_RMS) != 0);
+        at::head_rope(wave < LH ? s.tq[wave] : s.tk, inv, p.rw0, p.rw1, p.rc, p.rs,
+                      wave < LH ? s.qs[wave] : s.ks, lane);
+    }
+    __syncthreads();
+    if (xcd % 2 == 0 && rank == 0 && tid < at::HD) {
+        kg[(size_t)pos * at::KVD + tid] = s.ks[tid];
+        vg[(size_t)pos * at::KVD + tid] = s.tv[tid];
+    }
+    const int tl = tid / LH, hh = tid % LH;
+    for (int r0 = 0; r0 < p.cnt; r0 += LKR) {
+        const int m = min(LKR, p.cnt - r0);
+        if (r0) {
+            __syncthreads();  // the rows before are used
+            long_stage_keys(s, kg, p.t0 + r0, m, lane, wave);
+            __builtin_amdgcn_s_waitcnt(at::WAIT_VM0);
+            __syncthreads();
+        }
+        if (tl < m) {
+            const int t = p.t0 + r0 + tl;
+            const float dot = at::head_dot(s.qs[hh], (const float4 *)(t == pos ? s.ks : s.k[tl]));
+            put_tagged<true>(&xw->sc[xcd][hh][t], dot * a.scale, tag);
+        }
+    }
+}
+
+// Head hh of the XCD, elements LEL qt .. of it, by a workgroup; sc: pos + 1
+// floats of LDS, rounded up to a multiple of 4. `before_mix` runs once the
+// scores are in.
+template <class F>
+__device__ __forceinline__ void long_mix(const DecodeArgs &a, LongLds &s, DecodeWs *ws, float *sc,
+                                         at::gptr<const float> vg, const uint64_t *etab, int xcd,
+                                         int hh, int qt, int tid, int lane, int wave, unsigned tag,
+                                         F &&before_mix) {
+    const int pos = a.pos, n = pos + 1, h = LH * xcd + hh;
+    AttnXWs *xw = a.xw;
+    const tw *w = xw->sc[xcd][hh];
+    float mx = -__builtin_inff();
+    int b = 0;
+    for (; b + 4 * NT <= n; b += 4 * NT) {
+        float v[4];
+        get_tagged<4, true>(ws, w + b + tid, NT, tag, v);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            sc[b + tid + NT * k] = v[k];
+            mx = fmaxf(mx, v[k]);  // (keeps the larger of a number and a NaN)
+        }
+    }
+    for (int t = b + tid; t < n; t += NT) {
+        float v;
+        get_tagged<1, true>(ws, w + t, 0, tag, &v);
+        sc[t] = v;
+        mx = fmaxf(mx, v);
+    }
+    before_mix();
+    mx = at::max64(mx);
+    if (lane == 0) s.red[wave] = mx;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NWAVE; k++) mx = fmaxf(mx, s.red[k]);
+    for (int t = tid; t < n; t += NT) sc[t] = mia_expf_glibc_tab(sc[t] - mx, etab);
+    __syncthreads();
+    if (wave == 0) {
+        float sum = 0.0f;
+        int t = 0;
+        for (; t + 64 <= n; t += 64) sum = lds_seq_sum_pipe<64, 32>(sc + t, sum);
+        for (; t < n; t++) sum = sum + sc[t];
+        if (lane == 0) s.sum = sum;
+    }
+    // producers: slot (wave - 1) * 2 + lane / 32 + 14 u of the ring buffer,
+    // i.e. positions LC c + 4 slot .. + 3 of element lane % 32
+    const int el = lane & (LEL - 1), slot0 = (wave - 1) * 2 + (lane >> 5);
+    const at::gptr<const float> vp = vg + LEL * qt + el;
+    float vr[LU][4];
+    auto fetch = [&](int c) {
+#pragma unroll
+        for (int u = 0; u < LU; u++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                vr[u][j] = vp[(size_t)min(LC * c + 4 * (slot0 + 14 * u) + j, pos) * at::KVD];
+    };
+    static_assert(2 * (NWAVE - 1) == 14, "slots of a round");
+    if (wave) fetch(0);
+    __syncthreads();
+    const float sum = s.sum;
+    for (int t = tid; t < n; t += NT) sc[t] = sc[t] / sum;
+    __syncthreads();
+    float o = 0.0f;
+    const float vnew = s.tv[LEL * qt + el];
+    const int nc = (n + LC - 1) / LC;
+    if (wave == 0) __builtin_amdgcn_s_setprio(2);
+    for (int c = 0; c <= nc; c++) {
+        if (wave == 0) {
+            if (c) {
+                const float4 *r = &s.ring[(c - 1) & 1][0][el];
+                constexpr int B = 7;
+                static_assert(LSLOT % (2 * B) == 0, "whole rounds");
+                float4 x[B], y[B];
+#pragma unroll
+                for (int k = 0; k < B; k++) x[k] = r[k * LEL];
+#pragma unroll 1
+                for (int q = 0; q < LSLOT; q += 2 * B) {
+#pragma unroll
+                    for (int k = 0; k < B; k++) y[k] = r[(q + B + k) * LEL];
+#pragma unroll
+                    for (int k = 0; k < B; k++) {
+                        o = o + x[k].x;
+                        o = o + x[k].y;
+                        o = o + x[k].z;
+                        o = o + x[k].w;
+                    }
+                    const int qn = q + 2 * B < LSLOT ? q + 2 * B : 0;  // (last round: not used)
+#pragma unroll
+                    for (int k = 0; k < B; k++) x[k] = r[(qn + k) * LEL];
+#pragma unroll
+                    for (int k = 0; k < B; k++) {
+                        o = o + y[k].x;
+                        o = o + y[k].y;
+                        o = o + y[k].z;
+                        o = o + y[k].w;
+                    }
+                }
+            }
+        } else if (c < nc) {
+#pragma unroll
+            for (int u = 0; u < LU; u++) {
+                // (positions past the end: +0, which leaves a sum that
+                // started at +0 as it is)
+                const int slot = slot0 + 14 * u, t = LC * c + 4 * slot;
+                float4 pr = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                if (t < n) {
+                    const float4 p = *(const float4 *)&sc[t];
+                    pr.x = p.x * (t == pos ? vnew : vr[u][0]);
+                    if (t + 1 < n) pr.y = p.y * (t + 1 == pos ? vnew : vr[u][1]);
+                    if (t + 2 < n) pr.z = p.z * (t + 2 == pos ? vnew : vr[u][2]);
+                    if (t + 3 < n) pr.w = p.w * (t + 3 == pos ? vnew : vr[u][3]);
+                }
+                s.ring[c & 1][slot][el] = pr;
+            }
+            fetch(min(c + 1, nc - 1));
+        }
+        __syncthreads();
+    }
+    if (wave == 0) {
+        __builtin_amdgcn_s_setprio(0);
+        // Q8 of the 32 elements (one block; both half wavefronts hold them)
+        const float am = at::max32(fmaxf(0.0f, fabsf(o)), lane);  // a NaN counts as 0
+        const float d = am / 127.0f;
+        const float qi = d != 0.0f ? 1.0f / d : 0.0f;
+        if (lane < LEL) s.hq[lane] = (int8_t)roundf(o * qi);
+        wave_lds_sync();
+        if (lane < LEL / 4)
+            put_tagged<false>(&xw->attq[(h * at::HD + LEL * qt) / 4 + lane],
+                              __uint_as_float(((const unsigned *)s.hq)[lane]), tag);
+        if (lane == 0) put_tagged<false>(&xw->atts[h * LQT + qt], d, tag);
+    }
+}
+
 // `before_x` runs once the Wo rows are published, before the new x is
 // waited for: the caller's requests for the MoE that follows go there.
-template <class F>
+template <bool LONG, class F>
 __device__ __forceinline__ void attn_stage(const DecodeArgs &a, Lds &sh, DecodeWs *ws, int tid,
                                            int lane, int wave, int xcd, int rank, int l,
                                            unsigned tag, F &&before_x) {
@@ -581,7 +843,10 @@ __device__ __forceinline__ void attn_stage(const DecodeArgs &a, Lds &sh, DecodeW
     // layer rather than held across the loop (the place is made opaque): the
     // registers they would hold are what the MoE stages need.
     asm volatile("" : "+s"(xcd), "+s"(rank), "+s"(wave));
-    __shared__ at::HeadLds<AT_NPRE> hs;
+    // (the context's length chooses the kernel, and each holds only its own)
+    using HeadL = std::conditional_t<LONG, LongLds, at::HeadLds<AT_NPRE>>;
+    using HeadP = std::conditional_t<LONG, LongPre, at::HeadPre<AT_NPRE, true>>;
+    __shared__ HeadL hs;
     __shared__ alignas(16) int8_t attq[at::QD];
     __shared__ float atts[at::NBO];
     __shared__ mhip_attn_layer al_next;             // the next layer's tensors, read a layer ahead
@@ -629,8 +894,14 @@ __device__ __forceinline__ void attn_stage(const DecodeArgs &a, Lds &sh, DecodeW
     // critical path, then do not share HBM with the Wo rows.
     const at::gptr<const uint8_t> wo = wog + (size_t)gw * at::NBO * 36;
     at::Blk wo0, wo1;
-    at::HeadPre<AT_NPRE, true> hp;
-    if (head)
+    HeadP hp;
+    const int gx = LONG ? xcd / 2 : 0;  // (long contexts: the XCD's key/value group)
+    const at::gptr<float> kg = kcg + gx * at::HD, vg = vcg + gx * at::HD;
+    if constexpr (LONG)
+        long_prefetch(hp, hs, rank, a.pos, (at::gptr<const float>)kg, (at::gptr<const float>)vg,
+                      at::glob(uniform_ptr(L.q_norm)), at::glob(uniform_ptr(L.k_norm)),
+                      at::glob(a.rope), tid, lane, wave);
+    else if (head)
         at::head_prefetch(hp, hs, h, a.pos, (at::gptr<const float>)kcg, (at::gptr<const float>)vcg,
                           at::glob(uniform_ptr(L.q_norm)), at::glob(uniform_ptr(L.k_norm)),
                           at::glob(a.rope), tid);
@@ -716,13 +987,23 @@ __device__ __forceinline__ void attn_stage(const DecodeArgs &a, Lds &sh, DecodeW
         }
     }
     TRACE_BY(26, 63);
-    if (!head) {
+    auto load_wo = [&]() {
         wo0 = at::load_blk(wo + (size_t)lane * 36);
         wo1 = at::load_blk(wo + (size_t)(lane + 64) * 36);
-    }
+    };
+    if (!LONG && !head) load_wo();
 
     // query head h (forward.c:127-163)
-    if (head) {
+    if constexpr (LONG) {
+        long_scores(a, hs, ws, hp, kg, vg, xcd, rank, tid, lane, wave, tag);
+        TRACE(27);
+        if (rank < LH * LQT)
+            long_mix(a, hs, ws, asc, (at::gptr<const float>)vg, sh.etab, xcd, rank / LQT, rank % LQT,
+                     tid, lane, wave, tag, load_wo);
+        else
+            load_wo();
+        TRACE(28);
+    } else if (head) {
         const int g = h / at::GROUP;
         float v;
         if (tid < at::HD) {
@@ -745,8 +1026,7 @@ __device__ __forceinline__ void attn_stage(const DecodeArgs &a, Lds &sh, DecodeW
         if (tid < at::HD / 4)
             put_tagged<false>(&xw->attq[h * (at::HD / 4) + tid],
                               __uint_as_float(((const unsigned *)hs.hq)[tid]), tag);
-        wo0 = at::load_blk(wo + (size_t)lane * 36);
-        wo1 = at::load_blk(wo + (size_t)(lane + 64) * 36);
+        load_wo();
     }
 
     // row gw of Wo over the heads' codes, plus the residual (forward.c:164-165)
@@ -812,6 +1092,13 @@ __global__ __launch_bounds__(NT) void k_model_stack(DecodeArgs a) {
 #include "decode_body.inc"
 #undef DECODE_ATTN
 }
+__global__ __launch_bounds__(NT) void k_model_stack_long(DecodeArgs a) {
+#define DECODE_ATTN 2
+#include "decode_body.inc"
+#undef DECODE_ATTN
+}
+// Positions from which the heads are spread over their XCD.
+constexpr int LONG_MIN_POS = 128;
 
 // Once per context (the device properties query is slow): 1 when every CU
 // holds one workgroup of the kernel, 0 when not (c->decode_cus and
@@ -928,8 +1215,11 @@ int launch_decode(mhip_ctx *c, const mhip_dims *s, const mhip_layout *lay, const
     // resident at once. Should one not be, the start barrier times out and
     // the launch reports abort bit 2 instead of waiting for ever.
     int slot = mhip::stage_begin(c, MHIP_STAGE_DECODE);
-    if (mp)  // a head's scores in dynamic LDS
-        k_model_stack<<<NWG, NT, ((size_t)mp->pos + 1) * 4, c->stream>>>(a);
+    const size_t sc = mp ? (((size_t)mp->pos + 4) & ~(size_t)3) * 4 : 0;  // a head's scores
+    if (mp && mp->pos >= LONG_MIN_POS)
+        k_model_stack_long<<<NWG, NT, sc, c->stream>>>(a);
+    else if (mp)
+        k_model_stack<<<NWG, NT, sc, c->stream>>>(a);
     else
         k_decode_stack<<<NWG, NT, 0, c->stream>>>(a);
     const hipError_t e = hipGetLastError();
@@ -945,16 +1235,16 @@ int launch_decode(mhip_ctx *c, const mhip_dims *s, const mhip_layout *lay, const
     return 0;
 }
 
-// The dynamic-LDS limit of k_model_stack (a head's scores), set once per
-// device.
+// The dynamic-LDS limit of the model stack's kernels (a head's scores), set
+// once per device.
 int g_model_lds_set[MAX_DEVICES];
 int model_lds_attr(mhip_ctx *c) {
     if (c->device < 0 || c->device >= MAX_DEVICES || g_model_lds_set[c->device]) return 0;
-    if (mhip::check(c, hipFuncSetAttribute((const void *)k_model_stack,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           MHIP_MODEL_STACK_MAX_SEQ * 4),
-                    "model stack LDS attribute"))
-        return -1;
+    for (const void *k : {(const void *)k_model_stack, (const void *)k_model_stack_long})
+        if (mhip::check(c, hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                               MHIP_MODEL_STACK_MAX_SEQ * 4),
+                        "model stack LDS attribute"))
+            return -1;
     g_model_lds_set[c->device] = 1;
     return 0;
 }
@@ -1068,13 +1358,16 @@ int mhip_model_stack_supported(mhip_ctx *c, const mhip_dims *s, const mhip_attn_
     if (max_seq <= 0 || max_seq > MHIP_MODEL_STACK_MAX_SEQ) return 0;
     const int fits = decode_device_fits(c);
     if (fits <= 0) return fits;
-    int occ = 0;
-    if (model_lds_attr(c) ||
-        mhip::check(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_model_stack, NT,
-                                                                     (size_t)max_seq * 4),
+    if (model_lds_attr(c)) return -1;
+    const size_t lds = (((size_t)max_seq + 3) & ~(size_t)3) * 4;
+    int occ = 0, occ_long = 0;
+    if (mhip::check(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_model_stack, NT, lds),
+                    "occupancy") ||
+        mhip::check(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ_long, k_model_stack_long,
+                                                                     NT, lds),
                     "occupancy"))
         return -1;
-    return occ >= 1 ? 1 : 0;
+    return occ >= 1 && occ_long >= 1 ? 1 : 0;
 }
 
 int mhip_model_stack(mhip_ctx *c, const mhip_dims *s, const mhip_layout *lay,

@@ -364,3 +364,30 @@ def test_model_full_shape_prefill_far_positions():
     finally:
         a.close()
         b.close()
+
+
+def test_model_stack_long_contexts():
+    """Positions from which the model stack spreads a head over its XCD, on a
+    context filled by a prompt: around the switch (position 128), the ends of
+    the mix's 168-position buffers, of a workgroup's 80 staged key rows (a
+    32nd of 2560 positions), of the scores' 2048-word reads, and the longest
+    context; stack == one launch per layer (bits)."""
+    say("test_model_stack_long_contexts")
+    n = M.MHIP_MODEL_STACK_MAX_SEQ
+    cfg = dict(QWEN_FULL, n_layers=2, vocab=4000)
+    m = M.GpuModel(None, n, synth=(cfg, 17))
+    try:
+        rng = np.random.default_rng(15)
+        m.prefill(rng.integers(0, cfg["vocab"], n - 1).tolist(), 0)
+        for p in (n - 1, 5375, 5119, 4096, 4095, 2560, 2559, 2047, 671, 672, 503, 336, 335, 168, 167,
+                  160, 159, 129, 128, 127):
+            tok = int(rng.integers(0, cfg["vocab"]))
+            m.set_flags(EXACT | PER_LAYER)
+            want = m.step(tok, p).copy()
+            m.set_flags(EXACT)
+            got = m.step(tok, p)
+            assert m.aborts() == 0
+            assert np.all(np.isfinite(got))
+            assert np.array_equal(bits(got), bits(want)), "position %d" % p
+    finally:
+        m.close()
