@@ -63,6 +63,9 @@ __device__ __forceinline__ void dma4(unsigned lds, const void *g) {
     asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(g)
                  : "memory", "m0");
 }
+template <int N> __device__ __forceinline__ void wait_vm() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
 #pragma clang diagnostic pop
 
 // A DPP move of x (lanes of rows outside ROWS keep their own value, resp. 0

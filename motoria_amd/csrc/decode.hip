@@ -138,7 +138,9 @@ struct AttnXWs {
     alignas(256) tw atts[at::NBO];     // their block scales
     alignas(256) tw xa[D];             // x after the attention
     alignas(256) tw xl[NX][D];         // the same, republished in each XCD's L2
-    // long contexts: the scores of each XCD's four query heads
+    // long contexts: q, k, v of each XCD's four query heads and their group,
+    // and the heads' scores
+    alignas(256) tw ql[NX][(at::NH / NX + 2) * at::HD];
     alignas(256) tw sc[NX][at::NH / NX][MHIP_MODEL_STACK_MAX_SEQ];
 };
 
@@ -582,15 +584,16 @@ template <class T> __device__ __forceinline__ T *uniform_ptr(T *p) {
 // the positions for the four heads (its key rows copied into LDS while the
 // q/k/v rows form) and publishes the scores in the XCD's L2; workgroups of
 // rank < 16 then take a head and 32 of its elements each: softmax, and the
-// position-ordered mix as a pipeline: wavefronts 1-7 form the products
-// p_t v_t of LC positions in an LDS ring, from which wavefront 0 adds the
-// previous LC's, four to a read, so that the chain of one addition per
-// position (~5 cycles) is all that is serial. Every value and its order are
-// head_run's.
+// position-ordered mix as a pipeline: wavefronts 1-7 copy value rows into
+// LDS two steps ahead and form the products p_t v_t of LC positions in an
+// LDS ring, from which wavefront 0 adds the previous LC's, four to a read, so
+// that the chain of one addition per position (~5 cycles) is all that is
+// serial. Every value and its order are head_run's.
 constexpr int LH = at::NH / NX;        // query heads of an XCD
 constexpr int LKR = 80;                // key rows a workgroup stages at a time
 constexpr int LQ = at::HD + 4;         // q row stride
-constexpr int LU = 3;                  // four-position slots of a producer's half wavefront
+constexpr int LU = 2;                  // four-position slots of a producer's half wavefront
+constexpr int LVS = 3;                 // stages of its value rows
 constexpr int LSLOT = (NWAVE - 1) * 2 * LU, LC = 4 * LSLOT;  // slots, positions of a ring buffer
 constexpr int LEL = 32, LQT = at::HD / LEL;  // elements of a mixing workgroup, such parts of a head
 static_assert(LH * LQT <= WPX && LH == 4 && at::GROUP == 2 * LH, "a head's four parts on its XCD");
@@ -600,10 +603,10 @@ struct LongLds {
     alignas(16) float tk[at::HD], ks[at::HD], tv[at::HD];
     union alignas(16) {
         float k[LKR][at::KLD];              // staged key rows
-        float4 ring[2][LSLOT][LEL];          // products of four positions of an element
+        float v[NWAVE - 1][LVS][LU][8][LEL];  // each producer's value rows
     };
     float touch[64];                        // (target of the value rows' requests)
-    float red[NWAVE], inv[LH + 1], sum;
+    float red[NWAVE];
     alignas(16) int8_t hq[LEL];
 };
 
@@ -621,6 +624,11 @@ __device__ __forceinline__ void long_stage_keys(LongLds &s, at::gptr<const float
         else if (2 * q + 1 < m) at::dma16(k1, src);
     }
 }
+
+// The products of four positions of an element each.
+struct RingLds {
+    float4 p[2][LSLOT][LEL];
+};
 
 struct LongPre : at::HeadRope {
     int t0, cnt;  // this workgroup's positions
@@ -651,28 +659,28 @@ __device__ __forceinline__ void long_prefetch(LongPre &p, LongLds &s, int rank, 
 
 // The part of the heads that every workgroup does: q (and the new k) normed
 // and rotated, the cache rows appended, this workgroup's scores published.
+template <class Mark>
 __device__ __forceinline__ void long_scores(const DecodeArgs &a, LongLds &s, DecodeWs *ws,
                                             const LongPre &p, at::gptr<float> kg,
                                             at::gptr<float> vg, int xcd, int rank, int tid, int lane,
-                                            int wave, unsigned tag) {
-    const int g = xcd / 2, pos = a.pos;
+                                            int wave, unsigned tag, Mark mark) {
+    const int pos = a.pos;
     AttnXWs *xw = a.xw;
     {
         // q of the four heads (a word per thread), then k and v of the group
         float v[2];
         if (tid < 2 * at::HD) {
-            const int kv = at::QD + (tid < at::HD ? 0 : at::KVD - at::HD) + g * at::HD + tid;
-            get_tagged<2, false>(ws, &xw->qkv[LH * at::HD * xcd + tid],
-                                 kv - (LH * at::HD * xcd + tid), tag, v);
+            get_tagged<2, true>(ws, &xw->ql[xcd][tid], LH * at::HD, tag, v);
             if (tid < at::HD) s.tk[tid] = v[1];
             else s.tv[tid - at::HD] = v[1];
         } else {
-            get_tagged<1, false>(ws, &xw->qkv[LH * at::HD * xcd + tid], 0, tag, v);
+            get_tagged<1, true>(ws, &xw->ql[xcd][tid], 0, tag, v);
         }
         s.tq[tid / at::HD][tid % at::HD] = v[0];
     }
     __builtin_amdgcn_s_waitcnt(at::WAIT_VM0);  // this wavefront's key rows are in
     __syncthreads();
+    mark(6);
     if (wave <= LH) {
         const float inv = at::head_inv_wave(wave < LH ? s.tq[wave] : s.tk, a.eps, lane,
                                             (a.flags & MHIP_FORCE_SEQ_RMS) != 0);
@@ -680,6 +688,7 @@ __device__ __forceinline__ void long_scores(const DecodeArgs &a, LongLds &s, Dec
                       wave < LH ? s.qs[wave] : s.ks, lane);
     }
     __syncthreads();
+    mark(7);
     if (xcd % 2 == 0 && rank == 0 && tid < at::HD) {
         kg[(size_t)pos * at::KVD + tid] = s.ks[tid];
         vg[(size_t)pos * at::KVD + tid] = s.tv[tid];
@@ -701,14 +710,168 @@ __device__ __forceinline__ void long_scores(const DecodeArgs &a, LongLds &s, Dec
     }
 }
 
+// A run of fp32 additions s <- fl(s + v), v >= 0, inside one binade of s, as
+// the map of s's bits it is: there s = M u on a grid of spacing u, fl(s + v)
+// = (M + k) u with k the integer nearest v / u, and a tie goes to the even
+// M + k, so what is added to the bits depends on their lowest one alone.
+struct Run {
+    int a0, a1;  // added to even (odd) bits
+};
+__device__ __forceinline__ Run then(Run a, Run b) {
+    return {a.a0 + ((a.a0 & 1) ? b.a1 : b.a0), a.a1 + ((a.a1 & 1) ? b.a0 : b.a1)};
+}
+// The runs of the lanes before and this one, from the last lane that has
+// `head` set on (its own run included).
+template <int CTRL, int ROWS, bool ZERO_FILL>
+__device__ __forceinline__ void run_scan_step(Run &r, int &head) {
+    const Run p = {__builtin_amdgcn_update_dpp(0, r.a0, CTRL, ROWS, 0xf, ZERO_FILL),
+                   __builtin_amdgcn_update_dpp(0, r.a1, CTRL, ROWS, 0xf, ZERO_FILL)};
+    const int ph = __builtin_amdgcn_update_dpp(0, head, CTRL, ROWS, 0xf, ZERO_FILL);
+    if (!head) {
+        r = then(p, r);
+        head = ph;
+    }
+}
+
+// The reference's left-to-right fp32 sum of the n values e (LDS, e >= 0 or
+// NaN) by a workgroup, in every thread, without its chain of n additions:
+// each thread takes a piece of m values. The sequential sum at any point is
+// within n 2^-23 (relative) of the exact one, which the threads have from a
+// double scan; where that places a piece inside one binade of the running
+// sum, its additions are a Run. Runs compose, so a wavefront composes its
+// pieces between the others (the first, those at a power of two; about ten
+// of 512), and wavefront 0 walks what is left: a run's map, a piece's own
+// additions, and so on. Measured over 2501 values: 7.5 -> 2 us.
+constexpr int SM = 16;  // values of a piece, at most
+static_assert(SM * NT >= MHIP_MODEL_STACK_MAX_SEQ, "pieces");
+struct SumLds {
+    Run run[NT];
+    double part[NWAVE];
+    unsigned long long own[NWAVE];  // pieces added one value at a time
+    float sum;
+};
+__device__ __forceinline__ float block_seq_sum(const float *e, int n, SumLds &s, int tid, int lane,
+                                               int wave) {
+    const int m = 4 * ((n + 4 * NT - 1) / (4 * NT));
+    // the values of piece k, four at a time (+0 past the end)
+    float4 v[SM / 4];
+    auto load = [&](int k) {
+#pragma unroll
+        for (int j = 0; j < SM / 4; j++) {
+            const int t = k * m + 4 * j;
+            v[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (4 * j < m && t < n) {
+                v[j] = *(const float4 *)(e + t);
+                if (t + 1 >= n) v[j].y = 0.0f;
+                if (t + 2 >= n) v[j].z = 0.0f;
+                if (t + 3 >= n) v[j].w = 0.0f;
+            }
+        }
+    };
+    load(tid);
+    double own = 0.0;
+#pragma unroll
+    for (int j = 0; j < SM / 4; j++)
+        own = own + (((double)v[j].x + (double)v[j].y) + ((double)v[j].z + (double)v[j].w));
+    const double incl = wave_scan_d(own);
+    if (lane == 63) s.part[wave] = incl;
+    __syncthreads();
+    double base = 0.0;
+#pragma unroll
+    for (int k = 0; k < NWAVE; k++) base = base + (k < wave ? s.part[k] : 0.0);
+    const double S1 = base + incl, S0 = S1 - own, dl = (double)(n + 64) * 0x1p-23;
+    const unsigned b0 = (unsigned)((uint64_t)__double_as_longlong(S0 * (1.0 - dl)) >> 52);
+    const unsigned b1 = (unsigned)((uint64_t)__double_as_longlong(S1 * (1.0 + dl)) >> 52);
+    const bool zero = own == 0.0;  // (every value is +0: the sum stays)
+    const bool in = zero || (b0 == b1 && b0 >= 1023 - 100 && b0 < 1023 + 100);
+    Run r = {0, 0};
+    if (in && !zero) {
+        // v / u, u = 2^(P - 23), P = b0 - 1023: exact, or too small to count
+        const float scale = __int_as_float((int)(127 + 23 + 1023 - b0) << 23);
+        auto add1 = [&](float x) {
+            const float q = x * scale, f = floorf(q), fr = q - f;
+            const int k = (int)f, up = fr > 0.5f ? 1 : 0;
+            const bool tie = fr == 0.5f;
+            r.a0 = r.a0 + k + (tie ? (r.a0 + k) & 1 : up);
+            r.a1 = r.a1 + k + (tie ? (r.a1 + k + 1) & 1 : up);
+        };
+#pragma unroll
+        for (int j = 0; j < SM / 4; j++) {
+            if (4 * j < m) {
+                add1(v[j].x);
+                add1(v[j].y);
+                add1(v[j].z);
+                add1(v[j].w);
+            }
+        }
+    }
+    const unsigned long long mask = __ballot(!in);
+    int head = in ? 0 : 1;
+    run_scan_step<0x111, 0xf, true>(r, head);
+    run_scan_step<0x112, 0xf, true>(r, head);
+    run_scan_step<0x114, 0xf, true>(r, head);
+    run_scan_step<0x118, 0xf, true>(r, head);
+    run_scan_step<0x142, 0xa, false>(r, head);
+    run_scan_step<0x143, 0xc, false>(r, head);
+    s.run[tid] = r;
+    if (lane == 0) s.own[wave] = mask;
+    __syncthreads();
+    if (wave == 0) {
+        float sum = 0.0f;
+        auto apply = [&](int a0, int a1) {
+            const int b = __float_as_int(sum);
+            sum = __int_as_float(b + ((b & 1) ? a1 : a0));
+        };
+        auto lane_f = [](float x, int i) {
+            return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), i));
+        };
+        // the wavefronts' last lanes' runs, and their masks, read together
+        const Run last = s.run[min(64 * lane + 63, NT - 1)];
+        const unsigned long long own_l = s.own[min(lane, NWAVE - 1)];
+        for (int w = 0; w < NWAVE && 64 * w * m < n; w++) {
+            unsigned long long left =
+                (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(unsigned)own_l, w) |
+                (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(own_l >> 32), w) << 32;
+            int prev = -1;
+            if (left) {
+                // this wavefront's runs and values, a piece per lane
+                r = s.run[64 * w + lane];
+                load(64 * w + lane);
+                while (left) {
+                    const int i = __builtin_ctzll(left);
+                    left &= left - 1;
+                    if (i - 1 > prev)
+                        apply(__builtin_amdgcn_readlane(r.a0, i - 1),
+                              __builtin_amdgcn_readlane(r.a1, i - 1));
+#pragma unroll
+                    for (int j = 0; j < SM / 4; j++) {
+                        if (4 * j < m) {
+                            sum = sum + lane_f(v[j].x, i);
+                            sum = sum + lane_f(v[j].y, i);
+                            sum = sum + lane_f(v[j].z, i);
+                            sum = sum + lane_f(v[j].w, i);
+                        }
+                    }
+                    prev = i;
+                }
+            }
+            if (prev < 63)
+                apply(__builtin_amdgcn_readlane(last.a0, w), __builtin_amdgcn_readlane(last.a1, w));
+        }
+        if (lane == 0) s.sum = sum;
+    }
+    __syncthreads();
+    return s.sum;
+}
+
 // Head hh of the XCD, elements LEL qt .. of it, by a workgroup; sc: pos + 1
 // floats of LDS, rounded up to a multiple of 4. `before_mix` runs once the
-// scores are in.
-template <class F>
-__device__ __forceinline__ void long_mix(const DecodeArgs &a, LongLds &s, DecodeWs *ws, float *sc,
+// scores are in; mark(i), i = 0..5, after each phase (a phase trace).
+template <class F, class Mark>
+__device__ __forceinline__ void long_mix(const DecodeArgs &a, LongLds &s, float *scr, DecodeWs *ws, float *sc,
                                          at::gptr<const float> vg, const uint64_t *etab, int xcd,
                                          int hh, int qt, int tid, int lane, int wave, unsigned tag,
-                                         F &&before_mix) {
+                                         F &&before_mix, Mark mark) {
     const int pos = a.pos, n = pos + 1, h = LH * xcd + hh;
     AttnXWs *xw = a.xw;
     const tw *w = xw->sc[xcd][hh];
@@ -729,53 +892,58 @@ __device__ __forceinline__ void long_mix(const DecodeArgs &a, LongLds &s, Decode
         sc[t] = v;
         mx = fmaxf(mx, v);
     }
+    mark(0);
     before_mix();
     mx = at::max64(mx);
     if (lane == 0) s.red[wave] = mx;
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < NWAVE; k++) mx = fmaxf(mx, s.red[k]);
+    mark(1);
+#pragma unroll 4
     for (int t = tid; t < n; t += NT) sc[t] = mia_expf_glibc_tab(sc[t] - mx, etab);
     __syncthreads();
-    if (wave == 0) {
-        float sum = 0.0f;
-        int t = 0;
-        for (; t + 64 <= n; t += 64) sum = lds_seq_sum_pipe<64, 32>(sc + t, sum);
-        for (; t < n; t++) sum = sum + sc[t];
-        if (lane == 0) s.sum = sum;
-    }
-    // producers: slot (wave - 1) * 2 + lane / 32 + 14 u of the ring buffer,
-    // i.e. positions LC c + 4 slot .. + 3 of element lane % 32
-    const int el = lane & (LEL - 1), slot0 = (wave - 1) * 2 + (lane >> 5);
-    const at::gptr<const float> vp = vg + LEL * qt + el;
-    float vr[LU][4];
+    mark(2);
+    // producers: slots (wave - 1) * 2 + lane / 32 + 14 u of the ring, i.e.
+    // positions LC c + 4 slot .. + 3 of element lane % 32: per u eight rows,
+    // which the wavefront copies into LDS with one instruction
+    const int el = lane & (LEL - 1), half = lane >> 5;
+    const unsigned vl = wave ? (unsigned)(uintptr_t)&s.v[wave - 1][0][0][0][0] : 0u;
     auto fetch = [&](int c) {
 #pragma unroll
-        for (int u = 0; u < LU; u++)
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-                vr[u][j] = vp[(size_t)min(LC * c + 4 * (slot0 + 14 * u) + j, pos) * at::KVD];
+        for (int u = 0; u < LU; u++) {
+            const int t = min(LC * c + 56 * u + 8 * (wave - 1) + (lane >> 3), pos);
+            at::dma16(__builtin_amdgcn_readfirstlane(vl + (unsigned)(((c % LVS) * LU + u) * 8 * LEL * 4)),
+                      (const float *)(vg + (size_t)t * at::KVD + LEL * qt + 4 * (lane & 7)));
+        }
     };
-    static_assert(2 * (NWAVE - 1) == 14, "slots of a round");
-    if (wave) fetch(0);
-    __syncthreads();
-    const float sum = s.sum;
+    static_assert(2 * (NWAVE - 1) == 14 && LVS == 3, "slots of a round");
+    const int nc = (n + LC - 1) / LC;
+    if (wave) {
+        fetch(0);
+        fetch(1);
+    }
+    const float sum = block_seq_sum(sc, n, *(SumLds *)scr, tid, lane, wave);
+    mark(3);
     for (int t = tid; t < n; t += NT) sc[t] = sc[t] / sum;
     __syncthreads();
+    mark(4);
+    RingLds &ring = *(RingLds *)scr;  // (the sum's use of it is over)
+    static_assert(sizeof(RingLds) <= SCR * 4 && sizeof(SumLds) <= SCR * 4, "scr");
     float o = 0.0f;
     const float vnew = s.tv[LEL * qt + el];
-    const int nc = (n + LC - 1) / LC;
     if (wave == 0) __builtin_amdgcn_s_setprio(2);
     for (int c = 0; c <= nc; c++) {
         if (wave == 0) {
             if (c) {
-                const float4 *r = &s.ring[(c - 1) & 1][0][el];
+                // the products of the previous buffer added in order
+                const float4 *r = &ring.p[(c - 1) & 1][0][el];
                 constexpr int B = 7;
                 static_assert(LSLOT % (2 * B) == 0, "whole rounds");
                 float4 x[B], y[B];
 #pragma unroll
                 for (int k = 0; k < B; k++) x[k] = r[k * LEL];
-#pragma unroll 1
+#pragma unroll
                 for (int q = 0; q < LSLOT; q += 2 * B) {
 #pragma unroll
                     for (int k = 0; k < B; k++) y[k] = r[(q + B + k) * LEL];
@@ -786,9 +954,10 @@ __device__ __forceinline__ void long_mix(const DecodeArgs &a, LongLds &s, Decode
                         o = o + x[k].z;
                         o = o + x[k].w;
                     }
-                    const int qn = q + 2 * B < LSLOT ? q + 2 * B : 0;  // (last round: not used)
+                    if (q + 2 * B < LSLOT) {
 #pragma unroll
-                    for (int k = 0; k < B; k++) x[k] = r[(qn + k) * LEL];
+                        for (int k = 0; k < B; k++) x[k] = r[(q + 2 * B + k) * LEL];
+                    }
 #pragma unroll
                     for (int k = 0; k < B; k++) {
                         o = o + y[k].x;
@@ -799,25 +968,33 @@ __device__ __forceinline__ void long_mix(const DecodeArgs &a, LongLds &s, Decode
                 }
             }
         } else if (c < nc) {
+            fetch(c + 2);  // (into the stage used in step c - 1; rows past the end: row pos again)
+            at::wait_vm<2 * LU>();
 #pragma unroll
             for (int u = 0; u < LU; u++) {
-                // (positions past the end: +0, which leaves a sum that
-                // started at +0 as it is)
-                const int slot = slot0 + 14 * u, t = LC * c + 4 * slot;
-                float4 pr = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                if (t < n) {
-                    const float4 p = *(const float4 *)&sc[t];
-                    pr.x = p.x * (t == pos ? vnew : vr[u][0]);
-                    if (t + 1 < n) pr.y = p.y * (t + 1 == pos ? vnew : vr[u][1]);
-                    if (t + 2 < n) pr.z = p.z * (t + 2 == pos ? vnew : vr[u][2]);
-                    if (t + 3 < n) pr.w = p.w * (t + 3 == pos ? vnew : vr[u][3]);
+                const int slot = (wave - 1) * 2 + half + 14 * u, t = LC * c + 4 * slot;
+                const float *v = &s.v[wave - 1][c % LVS][u][4 * half][el];
+                const float4 p = *(const float4 *)&sc[min(t, pos & ~3)];
+                float4 pr;
+                pr.x = p.x * v[0];
+                pr.y = p.y * v[LEL];
+                pr.z = p.z * v[2 * LEL];
+                pr.w = p.w * v[3 * LEL];
+                if (t + 4 > pos) {
+                    // the new row; past it +0, which leaves a sum that started
+                    // at +0 as it is
+                    pr.x = t < pos ? pr.x : t == pos ? p.x * vnew : 0.0f;
+                    pr.y = t + 1 < pos ? pr.y : t + 1 == pos ? p.y * vnew : 0.0f;
+                    pr.z = t + 2 < pos ? pr.z : t + 2 == pos ? p.z * vnew : 0.0f;
+                    pr.w = t + 3 < pos ? pr.w : t + 3 == pos ? p.w * vnew : 0.0f;
                 }
-                s.ring[c & 1][slot][el] = pr;
+                ring.p[c & 1][slot][el] = pr;
             }
-            fetch(min(c + 1, nc - 1));
         }
         __syncthreads();
     }
+    if (wave) at::wait_vm<0>();
+    mark(5);
     if (wave == 0) {
         __builtin_amdgcn_s_setprio(0);
         // Q8 of the 32 elements (one block; both half wavefronts hold them)
@@ -882,11 +1059,21 @@ __device__ __forceinline__ void attn_stage(const DecodeArgs &a, Lds &sh, DecodeW
     at::Blk wr[AT_RPW];
 #pragma unroll
     for (int j = 0; j < AT_RPW; j++) {
-        const int r = min(gw + NWG * NWAVE * j, at::NROWS - 1);  // past the end: unused
-        const at::gptr<const uint8_t> w = r < at::QD ? wqg + (size_t)r * at::NB * 36
-                                          : r < at::QD + at::KVD
-                                              ? wkg + (size_t)(r - at::QD) * at::NB * 36
-                                              : wvg + (size_t)(r - at::QD - at::KVD) * at::NB * 36;
+        at::gptr<const uint8_t> w;
+        if constexpr (LONG) {
+            // the rows of the XCD's own heads: two of q, one of the group's k
+            // or v (which the group's other XCD forms as well: three rows a
+            // wavefront either way, and they stay inside the XCD)
+            const int wi = rank * NWAVE + wave, kv = xcd / 2 * at::HD + wi % at::HD;
+            w = j < 2 ? wqg + (size_t)(LH * at::HD * xcd + NWAVE * WPX * j + wi) * at::NB * 36
+                      : (wi < at::HD ? wkg : wvg) + (size_t)kv * at::NB * 36;
+            static_assert(AT_RPW == 3 && NWAVE * WPX == 2 * at::HD, "rows of an XCD");
+        } else {
+            const int r = min(gw + NWG * NWAVE * j, at::NROWS - 1);  // past the end: unused
+            w = r < at::QD ? wqg + (size_t)r * at::NB * 36
+                : r < at::QD + at::KVD ? wkg + (size_t)(r - at::QD) * at::NB * 36
+                                       : wvg + (size_t)(r - at::QD - at::KVD) * at::NB * 36;
+        }
         wr[j] = at::load_blk(w + (size_t)lane * 36);
     }
     // This wavefront's Wo row is requested once its q/k/v rows are in (and,
@@ -982,7 +1169,10 @@ __device__ __forceinline__ void attn_stage(const DecodeArgs &a, Lds &sh, DecodeW
 #pragma unroll
             for (int j = 0; j < AT_RPW; j++) {
                 const int r = gw + NWG * NWAVE * j;
-                if (r < at::NROWS) put_tagged<false>(&xw->qkv[r], sv[j], tag);
+                if constexpr (LONG)
+                    put_tagged<true>(&xw->ql[xcd][NWAVE * WPX * j + rank * NWAVE + wave], sv[j], tag);
+                else if (r < at::NROWS)
+                    put_tagged<false>(&xw->qkv[r], sv[j], tag);
             }
         }
     }
@@ -995,11 +1185,11 @@ __device__ __forceinline__ void attn_stage(const DecodeArgs &a, Lds &sh, DecodeW
 
     // query head h (forward.c:127-163)
     if constexpr (LONG) {
-        long_scores(a, hs, ws, hp, kg, vg, xcd, rank, tid, lane, wave, tag);
+        long_scores(a, hs, ws, hp, kg, vg, xcd, rank, tid, lane, wave, tag, [=](int i) { TRACE(38 + i); });
         TRACE(27);
         if (rank < LH * LQT)
-            long_mix(a, hs, ws, asc, (at::gptr<const float>)vg, sh.etab, xcd, rank / LQT, rank % LQT,
-                     tid, lane, wave, tag, load_wo);
+            long_mix(a, hs, sh.scr, ws, asc, (at::gptr<const float>)vg, sh.etab, xcd, rank / LQT, rank % LQT,
+                     tid, lane, wave, tag, load_wo, [=](int i) { TRACE(38 + i); });
         else
             load_wo();
         TRACE(28);
