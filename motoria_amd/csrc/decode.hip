@@ -587,8 +587,10 @@ template <class T> __device__ __forceinline__ T *uniform_ptr(T *p) {
 // position-ordered mix as a pipeline: wavefronts 1-7 copy value rows into
 // LDS two steps ahead and form the products p_t v_t of LC positions in an
 // LDS ring, from which wavefront 0 adds the previous LC's, four to a read, so
-// that the chain of one addition per position (~5 cycles) is all that is
-// serial. Every value and its order are head_run's.
+// that the chain of one addition per position is all that is serial (its
+// operands from LDS: 6.7 cycles an addition against 4.8 in registers).
+// Every value and its order are head_run's. At position 2500 a layer's
+// attention: scores ~3.5 us after q/k/v are out, softmax ~7, mix 9.4.
 constexpr int LH = at::NH / NX;        // query heads of an XCD
 constexpr int LKR = 80;                // key rows a workgroup stages at a time
 constexpr int LQ = at::HD + 4;         // q row stride
@@ -625,10 +627,15 @@ __device__ __forceinline__ void long_stage_keys(LongLds &s, at::gptr<const float
     }
 }
 
-// The products of four positions of an element each.
+// The products of four positions of an element each, and how far the
+// producers and the consumer are (steps done).
 struct RingLds {
     float4 p[2][LSLOT][LEL];
+    int made[NWAVE - 1], used;
 };
+__device__ __forceinline__ int lds_flag(const int *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
 
 struct LongPre : at::HeadRope {
     int t0, cnt;  // this workgroup's positions
@@ -741,7 +748,8 @@ __device__ __forceinline__ void run_scan_step(Run &r, int &head) {
 // sum, its additions are a Run. Runs compose, so a wavefront composes its
 // pieces between the others (the first, those at a power of two; about ten
 // of 512), and wavefront 0 walks what is left: a run's map, a piece's own
-// additions, and so on. Measured over 2501 values: 7.5 -> 2 us.
+// additions, and so on. Measured over 2501 values: 7.5 -> 4.6 us.
+constexpr int SUM_MIN_N = 320;  // below, the chain itself is faster (2.0 against 2.4 us at 201 values)
 constexpr int SM = 16;  // values of a piece, at most
 static_assert(SM * NT >= MHIP_MODEL_STACK_MAX_SEQ, "pieces");
 struct SumLds {
@@ -752,6 +760,52 @@ struct SumLds {
 };
 __device__ __forceinline__ float block_seq_sum(const float *e, int n, SumLds &s, int tid, int lane,
                                                int wave) {
+    if (n < SUM_MIN_N) {
+        if (wave == 0) {
+            // 32 values read ahead of their additions (+0 past the end)
+            constexpr int B = 8;
+            float4 x[B], y[B];
+            auto get = [&](float4 (&v)[B], int t) {
+#pragma unroll
+                for (int k = 0; k < B; k++) v[k] = *(const float4 *)(e + min(t + 4 * k, (n - 1) & ~3));
+            };
+            float sum = 0.0f;
+            auto add = [&](const float4 (&v)[B], int t) {
+                if (t + 4 * B <= n) {
+#pragma unroll
+                    for (int k = 0; k < B; k++) {
+                        sum = sum + v[k].x;
+                        sum = sum + v[k].y;
+                        sum = sum + v[k].z;
+                        sum = sum + v[k].w;
+                    }
+                } else {
+#pragma unroll
+                    for (int k = 0; k < B; k++) {
+                        const int d = n - t - 4 * k;
+                        sum = sum + (d > 0 ? v[k].x : 0.0f);
+                        sum = sum + (d > 1 ? v[k].y : 0.0f);
+                        sum = sum + (d > 2 ? v[k].z : 0.0f);
+                        sum = sum + (d > 3 ? v[k].w : 0.0f);
+                    }
+                }
+            };
+            // (the scheduler keeps the reads ahead of the additions)
+            get(x, 0);
+            for (int t = 0; t < n; t += 8 * B) {
+                get(y, t + 4 * B);
+                __builtin_amdgcn_sched_barrier(0);
+                add(x, t);
+                __builtin_amdgcn_sched_barrier(0);
+                get(x, t + 8 * B);
+                __builtin_amdgcn_sched_barrier(0);
+                add(y, t + 4 * B);
+            }
+            if (lane == 0) s.sum = sum;
+        }
+        __syncthreads();
+        return s.sum;
+    }
     const int m = 4 * ((n + 4 * NT - 1) / (4 * NT));
     // the values of piece k, four at a time (+0 past the end)
     float4 v[SM / 4];
@@ -926,77 +980,102 @@ __device__ __forceinline__ void long_mix(const DecodeArgs &a, LongLds &s, float 
     const float sum = block_seq_sum(sc, n, *(SumLds *)scr, tid, lane, wave);
     mark(3);
     for (int t = tid; t < n; t += NT) sc[t] = sc[t] / sum;
-    __syncthreads();
-    mark(4);
     RingLds &ring = *(RingLds *)scr;  // (the sum's use of it is over)
     static_assert(sizeof(RingLds) <= SCR * 4 && sizeof(SumLds) <= SCR * 4, "scr");
+    if (tid < NWAVE - 1) ring.made[tid] = 0;
+    if (tid == NWAVE - 1) ring.used = 0;
+    __syncthreads();
+    mark(4);
+    // No barriers in the pipeline: a producer writes step c into buffer c % 2
+    // once step c - 2 is used, then its count; the consumer reads on as far
+    // as the counts go. (A wavefront's LDS operations execute in order.
+    // Neither waits for anything but the other, so every wait ends.)
     float o = 0.0f;
-    const float vnew = s.tv[LEL * qt + el];
-    if (wave == 0) __builtin_amdgcn_s_setprio(2);
-    for (int c = 0; c <= nc; c++) {
-        if (wave == 0) {
-            if (c) {
-                // the products of the previous buffer added in order
-                const float4 *r = &ring.p[(c - 1) & 1][0][el];
-                constexpr int B = 7;
-                static_assert(LSLOT % (2 * B) == 0, "whole rounds");
-                float4 x[B], y[B];
+    if (wave == 0) {
+        __builtin_amdgcn_s_setprio(2);
+        constexpr int B = LSLOT / 2;
+        static_assert(LSLOT % 2 == 0, "two batches a step");
+        float4 x[B], y[B];
+        auto get = [&](float4 (&v)[B], int c, int q) {
+            const float4 *r = &ring.p[c & 1][q * B][el];
 #pragma unroll
-                for (int k = 0; k < B; k++) x[k] = r[k * LEL];
+            for (int k = 0; k < B; k++) v[k] = r[k * LEL];
+        };
+        auto add = [&](const float4 (&v)[B]) {
+            // (the reads before it stay ahead of the additions: left free, the
+            // compiler gathers a round's reads at its top and waits for them)
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int q = 0; q < LSLOT; q += 2 * B) {
-#pragma unroll
-                    for (int k = 0; k < B; k++) y[k] = r[(q + B + k) * LEL];
-#pragma unroll
-                    for (int k = 0; k < B; k++) {
-                        o = o + x[k].x;
-                        o = o + x[k].y;
-                        o = o + x[k].z;
-                        o = o + x[k].w;
-                    }
-                    if (q + 2 * B < LSLOT) {
-#pragma unroll
-                        for (int k = 0; k < B; k++) x[k] = r[(q + 2 * B + k) * LEL];
-                    }
-#pragma unroll
-                    for (int k = 0; k < B; k++) {
-                        o = o + y[k].x;
-                        o = o + y[k].y;
-                        o = o + y[k].z;
-                        o = o + y[k].w;
-                    }
-                }
+            for (int k = 0; k < B; k++) {
+                o = o + v[k].x;
+                o = o + v[k].y;
+                o = o + v[k].z;
+                o = o + v[k].w;
             }
-        } else if (c < nc) {
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto counts = [&]() { return lds_flag(&ring.made[min(lane, NWAVE - 2)]); };
+        while (__ballot(counts() < 1)) {}
+        wave_lds_sync();
+        get(x, 0, 0);
+        for (int c = 0; c < nc; c++) {
+            get(y, c, 1);
+            wave_lds_sync();  // (LDS takes the reads above before the count)
+            if (lane == 0)
+                __hip_atomic_store(&ring.used, c + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            int made = counts();  // (back by the end of the additions)
+            add(x);
+            const int next = min(c + 2, nc);
+            while (__ballot(made < next)) made = counts();
+            wave_lds_sync();
+            get(x, c + 1, 0);  // (after the last step: not used)
+            add(y);
+        }
+        __builtin_amdgcn_s_setprio(0);
+    } else {
+        const float vnew = s.tv[LEL * qt + el];
+        for (int c = 0; c < nc; c++) {
             fetch(c + 2);  // (into the stage used in step c - 1; rows past the end: row pos again)
             at::wait_vm<2 * LU>();
+            float4 p[LU], pr[LU];
+            int t[LU];
 #pragma unroll
             for (int u = 0; u < LU; u++) {
-                const int slot = (wave - 1) * 2 + half + 14 * u, t = LC * c + 4 * slot;
                 const float *v = &s.v[wave - 1][c % LVS][u][4 * half][el];
-                const float4 p = *(const float4 *)&sc[min(t, pos & ~3)];
-                float4 pr;
-                pr.x = p.x * v[0];
-                pr.y = p.y * v[LEL];
-                pr.z = p.z * v[2 * LEL];
-                pr.w = p.w * v[3 * LEL];
-                if (t + 4 > pos) {
+                t[u] = LC * c + 56 * u + 8 * (wave - 1) + 4 * half;
+                p[u] = *(const float4 *)&sc[min(t[u], pos & ~3)];
+                pr[u] = make_float4(v[0], v[LEL], v[2 * LEL], v[3 * LEL]);
+            }
+#pragma unroll
+            for (int u = 0; u < LU; u++) {
+                pr[u].x = p[u].x * pr[u].x;
+                pr[u].y = p[u].y * pr[u].y;
+                pr[u].z = p[u].z * pr[u].z;
+                pr[u].w = p[u].w * pr[u].w;
+                if (t[u] + 4 > pos) {
                     // the new row; past it +0, which leaves a sum that started
                     // at +0 as it is
-                    pr.x = t < pos ? pr.x : t == pos ? p.x * vnew : 0.0f;
-                    pr.y = t + 1 < pos ? pr.y : t + 1 == pos ? p.y * vnew : 0.0f;
-                    pr.z = t + 2 < pos ? pr.z : t + 2 == pos ? p.z * vnew : 0.0f;
-                    pr.w = t + 3 < pos ? pr.w : t + 3 == pos ? p.w * vnew : 0.0f;
+                    const int d = pos - t[u];
+                    pr[u].x = d > 0 ? pr[u].x : d == 0 ? p[u].x * vnew : 0.0f;
+                    pr[u].y = d > 1 ? pr[u].y : d == 1 ? p[u].y * vnew : 0.0f;
+                    pr[u].z = d > 2 ? pr[u].z : d == 2 ? p[u].z * vnew : 0.0f;
+                    pr[u].w = d > 3 ? pr[u].w : d == 3 ? p[u].w * vnew : 0.0f;
                 }
-                ring.p[c & 1][slot][el] = pr;
             }
+            while (lds_flag(&ring.used) < c - 1) {}
+            wave_lds_sync();
+#pragma unroll
+            for (int u = 0; u < LU; u++)
+                ring.p[c & 1][(wave - 1) * 2 + half + 14 * u][el] = pr[u];
+            wave_lds_sync();
+            if (lane == 0)
+                __hip_atomic_store(&ring.made[wave - 1], c + 1, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WORKGROUP);
         }
-        __syncthreads();
+        at::wait_vm<0>();
     }
-    if (wave) at::wait_vm<0>();
     mark(5);
     if (wave == 0) {
-        __builtin_amdgcn_s_setprio(0);
         // Q8 of the 32 elements (one block; both half wavefronts hold them)
         const float am = at::max32(fmaxf(0.0f, fabsf(o)), lane);  // a NaN counts as 0
         const float d = am / 127.0f;
@@ -1287,8 +1366,11 @@ __global__ __launch_bounds__(NT) void k_model_stack_long(DecodeArgs a) {
 #include "decode_body.inc"
 #undef DECODE_ATTN
 }
-// Positions from which the heads are spread over their XCD.
-constexpr int LONG_MIN_POS = 128;
+// Positions from which the heads are spread over their XCD: where a head's
+// workgroup has more cache rows than it stages in LDS. A step of the 48-layer
+// model, us, one workgroup a head / spread: position 8 1522/1669, 30
+// 1586/1670, 60 1971/1692, 100 1936/1665, 2500 9270/2450.
+constexpr int LONG_MIN_POS = AT_NPRE + 1;
 
 // Once per context (the device properties query is slow): 1 when every CU
 // holds one workgroup of the kernel, 0 when not (c->decode_cus and

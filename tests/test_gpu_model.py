@@ -368,10 +368,11 @@ def test_model_full_shape_prefill_far_positions():
 
 def test_model_stack_long_contexts():
     """Positions from which the model stack spreads a head over its XCD, on a
-    context filled by a prompt: around the switch (position 128), the ends of
-    the mix's 168-position buffers, of a workgroup's 80 staged key rows (a
-    32nd of 2560 positions), of the scores' 2048-word reads, and the longest
-    context; stack == one launch per layer (bits)."""
+    context filled by a prompt: around the switch (position 33), the ends of
+    the mix's 112-position buffers, the sum's two forms (320 values), a
+    workgroup's 80 staged key rows (a 32nd of 2560 positions), the scores'
+    2048-word reads, and the longest context; stack == one launch per layer
+    (bits)."""
     say("test_model_stack_long_contexts")
     n = M.MHIP_MODEL_STACK_MAX_SEQ
     cfg = dict(QWEN_FULL, n_layers=2, vocab=4000)
@@ -379,8 +380,8 @@ def test_model_stack_long_contexts():
     try:
         rng = np.random.default_rng(15)
         m.prefill(rng.integers(0, cfg["vocab"], n - 1).tolist(), 0)
-        for p in (n - 1, 5375, 5119, 4096, 4095, 2560, 2559, 2047, 671, 672, 503, 336, 335, 168, 167,
-                  160, 159, 129, 128, 127):
+        for p in (n - 1, 5375, 5119, 4096, 4095, 2560, 2559, 2047, 671, 672, 336, 335, 320, 319, 318,
+                  224, 223, 113, 112, 111, 64, 35, 34, 33, 32, 31):
             tok = int(rng.integers(0, cfg["vocab"]))
             m.set_flags(EXACT | PER_LAYER)
             want = m.step(tok, p).copy()
