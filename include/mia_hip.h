@@ -264,6 +264,14 @@ int mhip_decode_stack_noalloc(mhip_ctx *c, const mhip_dims *s, const mhip_layout
                               float *d_x, int L, int *d_idx, float *d_w, int *d_status,
                               int flags);
 int mhip_decode_status(mhip_ctx *c, const void *d_ws, int status[4]);
+/* A host call's x to the device, and a decode launch's results to the host,
+ * through pinned memory (mhip_host_malloc): one small launch each, the second
+ * with the call's one wait. mhip_decode_out leaves x [d], idx [nr], w [nr]
+ * (32-bit words, in this order) and six words of its own at h_out, and the
+ * launch's status as mhip_decode_status gives it. */
+int mhip_decode_in(mhip_ctx *c, float *d_x, const float *h_x, int d);
+int mhip_decode_out(mhip_ctx *c, const void *d_ws, const float *d_x, int d, const int *d_idx,
+                    const float *d_w, int nr, void *h_out, int status[4]);
 /* With MHIP_DECODE_TRACE set: the 100 MHz real-time counter read by thread 0
  * of each of the 256 workgroups at up to MHIP_TRACE_SLOTS stage boundaries
  * of layers MHIP_TRACE_L0 .. MHIP_TRACE_L0 + MHIP_TRACE_NL - 1

@@ -146,6 +146,8 @@ SIGNATURES = {
     "mhip_decode_stack_noalloc": (_i, [_p, ctypes.POINTER(Dims), ctypes.POINTER(Layout), _p, _p,
                                        _p, _p, _p, _p, _i, _p, _p, _p, _i]),
     "mhip_decode_status": (_i, [_p, _p, ctypes.POINTER(_i)]),
+    "mhip_decode_in": (_i, [_p, _p, _p, _i]),
+    "mhip_decode_out": (_i, [_p, _p, _p, _i, _p, _p, _i, _p, _p]),
     "mhip_decode_trace": (_i, [_p, _p, _p]),
     "mhip_attention_scratch_bytes": (_sz, [ctypes.POINTER(AttnDims), _i]),
     "mhip_attention": (_i, [_p, ctypes.POINTER(AttnDims), _p, _p, _p, _p, _p, _p, _p, _p, _p,

@@ -62,6 +62,7 @@
 // rmsnorm, Q/K/V rows, the 32 heads with the KV cache, Wo and the residual,
 // src/model/forward.c:118-165) before that layer's MoE, so a whole decode
 // token is one launch (forward.c:210-213).
+#include <cstring>
 #include <mutex>
 #include <type_traits>
 
@@ -1434,6 +1435,26 @@ __global__ void k_decode_status_out(const DecodeWs *ws, unsigned epoch, int *sta
     }
 }
 
+// A host call's x into the device buffer, and its results out of it, between
+// pinned host memory and the device: one small launch each way, where every
+// copy of the runtime's is a command of its own (a 1-layer call's five took
+// ~100 us of its 134).
+__global__ __launch_bounds__(256) void k_decode_in(float *__restrict__ x,
+                                                   const float *__restrict__ h, int d) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < d) x[i] = h[i];
+}
+__global__ __launch_bounds__(256) void k_decode_out(const DecodeWs *ws, const float *__restrict__ x,
+                                                    int d, const int *__restrict__ idx,
+                                                    const float *__restrict__ w, int nr,
+                                                    unsigned *__restrict__ h) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < d) h[i] = __float_as_uint(x[i]);
+    if (i < nr) h[d + i] = (unsigned)idx[i];
+    if (i < nr) h[d + nr + i] = __float_as_uint(w[i]);
+    if (i < 6) h[d + 2 * nr + i] = ((const unsigned *)ws->status)[i];
+}
+
 // One launch of the decode kernel on workspace ws, whose launches are
 // counted by *epoch. Exchanged words and status words are tagged with the
 // launch's epoch, so stale words of earlier launches never match, and the
@@ -1676,14 +1697,41 @@ int mhip_model_stack(mhip_ctx *c, const mhip_dims *s, const mhip_layout *lay,
     return rc;
 }
 
-int mhip_decode_status(mhip_ctx *c, const void *d_ws, int status[4]) {
-    const DecodeWs *ws = (const DecodeWs *)d_ws;
-    tw st[3];
-    if (mhip_d2h(c, st, ws->status, sizeof st)) return -1;
+// The launch's status from its tagged words.
+static void read_status(mhip_ctx *c, const void *d_ws, const tw *st, int status[4]) {
     for (int i = 0; i < 3; i++)
         status[i] = (d_ws == c->decode_ws && (unsigned)(st[i] >> 32) == c->decode_epoch)
                         ? (int)(unsigned)st[i] : 0;
     status[3] = 0;
+}
+
+int mhip_decode_status(mhip_ctx *c, const void *d_ws, int status[4]) {
+    const DecodeWs *ws = (const DecodeWs *)d_ws;
+    tw st[3];
+    if (mhip_d2h(c, st, ws->status, sizeof st)) return -1;
+    read_status(c, d_ws, st, status);
+    return 0;
+}
+
+int mhip_decode_in(mhip_ctx *c, float *d_x, const float *h_x, int d) {
+    if (d <= 0 || !d_x || !h_x) return mhip::fail(c, "decode in: bad arguments (d=%d)", d);
+    if (mhip::use_device(c)) return -1;
+    k_decode_in<<<mhip::blocks_for(d, 256), 256, 0, c->stream>>>(d_x, h_x, d);
+    return mhip::check_launch(c, "decode in");
+}
+
+int mhip_decode_out(mhip_ctx *c, const void *d_ws, const float *d_x, int d, const int *d_idx,
+                    const float *d_w, int nr, void *h_out, int status[4]) {
+    if (d <= 0 || nr < 0 || !d_ws || !d_x || !h_out)
+        return mhip::fail(c, "decode out: bad arguments (d=%d, nr=%d)", d, nr);
+    if (mhip::use_device(c)) return -1;
+    const int m = d > nr ? d : nr;
+    k_decode_out<<<mhip::blocks_for(m > 6 ? m : 6, 256), 256, 0, c->stream>>>(
+        (const DecodeWs *)d_ws, d_x, d, d_idx, d_w, nr, (unsigned *)h_out);
+    if (mhip::check_launch(c, "decode out") || mhip_sync(c)) return -1;
+    tw st[3];
+    memcpy(st, (const unsigned *)h_out + d + 2 * nr, sizeof st);
+    read_status(c, d_ws, st, status);
     return 0;
 }
 

@@ -23,7 +23,7 @@ struct mia_moe {
     float *d_router_dl; /* [L][E][dim], decode layout (mhip_router_decode_layout) */
     void *d_dws;        /* persistent decode workspace */
     int *d_didx;        /* [L][K] routing of the last decode-stack call */
-    float *h_stage;     /* pinned: x in [dim], x out [dim], idx [K], w [K] of one-token calls */
+    float *h_stage;     /* pinned: x in [dim], then mhip_decode_out's [dim + 2 L K + 6], of one-token calls */
     float *d_dw;        /* [L][K] */
     float *d_norm;      /* [L][dim] */
     float *d_router;    /* [E][dim] upload staging */
@@ -152,7 +152,7 @@ int mia_moe_open(mia_moe **out, const mia_moe_config *cfg, char *err, size_t err
         m->d_bias = mhip_malloc(m->gpu, E * 4);
         m->d_blob = mhip_malloc(m->gpu, m->blob_bytes);
         m->h_blob = malloc(m->blob_bytes);
-        m->h_stage = (float *)mhip_host_malloc(m->gpu, (2 * d + 2 * (size_t)cfg->n_active) * 4);
+        m->h_stage = (float *)mhip_host_malloc(m->gpu, (2 * d + 2 * (size_t)cfg->n_layers * cfg->n_active + 6) * 4);
         if (!m->d_table || !m->d_router_t || !m->d_router_dl || !m->d_dws || !m->d_didx ||
             !m->d_dw || !m->d_norm || !m->d_router || !m->d_scratch || !m->d_x || !m->d_bias ||
             !m->d_blob || !m->h_stage)
@@ -340,11 +340,18 @@ static int decode_per_stage(mia_moe *m, int l0, int l1, const float *d_bias) {
 int mia_moe_decode(mia_moe *m, int l0, int l1, float *x, const float *bias, int *idx, float *w) {
     const size_t d = (size_t)m->dims.dim, E = (size_t)m->dims.n_experts,
                  K = (size_t)m->dims.n_active;
-    if (mhip_h2d(m->gpu, m->d_x, x, d * 4)) return gpu_fail(m);
+    if (l0 < 0 || l1 > m->n_layers || l0 > l1)
+        return fail(m, "layer range [%d, %d) outside [0, %d)", l0, l1, m->n_layers);
+    const size_t nr = (size_t)(l1 - l0) * K;
+    float *hx = m->h_stage, *hy = m->h_stage + d;
+    memcpy(hx, x, d * 4);
+    if (mhip_decode_in(m->gpu, m->d_x, hx, (int)d)) return gpu_fail(m);
     if (bias && mhip_h2d(m->gpu, m->d_bias, bias, E * 4)) return gpu_fail(m);
     if (mia_moe_decode_dev(m, l0, l1, m->d_x, bias ? m->d_bias : NULL)) return -1;
     int st[4];
-    if (mhip_sync(m->gpu) || mhip_decode_status(m->gpu, m->d_dws, st)) return gpu_fail(m);
+    if (mhip_decode_out(m->gpu, m->d_dws, m->d_x, (int)d, m->d_didx + l0 * K, m->d_dw + l0 * K,
+                        (int)nr, hy, st))
+        return gpu_fail(m);
     if (st[0]) {
         /* The launch aborted (a wait timed out, workgroups not placed as it
          * needs, or a forced abort) and left d_x invalid; x (host) is
@@ -353,11 +360,14 @@ int mia_moe_decode(mia_moe *m, int l0, int l1, float *x, const float *bias, int 
         if (mhip_h2d(m->gpu, m->d_x, x, d * 4) ||
             decode_per_stage(m, l0, l1, bias ? m->d_bias : NULL))
             return -1;
+        int ignored[4];
+        if (mhip_decode_out(m->gpu, m->d_dws, m->d_x, (int)d, m->d_didx + l0 * K,
+                            m->d_dw + l0 * K, (int)nr, hy, ignored))
+            return gpu_fail(m);
     }
-    if (mhip_d2h(m->gpu, x, m->d_x, d * 4) ||
-        (idx && mhip_d2h(m->gpu, idx, m->d_didx + l0 * K, (size_t)(l1 - l0) * K * 4)) ||
-        (w && mhip_d2h(m->gpu, w, m->d_dw + l0 * K, (size_t)(l1 - l0) * K * 4)))
-        return gpu_fail(m);
+    memcpy(x, hy, d * 4);
+    if (idx) memcpy(idx, hy + d, nr * 4);
+    if (w) memcpy(w, hy + d + nr, nr * 4);
     return 0;
 }
 
@@ -379,19 +389,18 @@ static int check_status(mia_moe *m, int l0) {
 
 /* One token through one layer in a launch of the persistent decode kernel
  * with the exact router (bit-equal to the reference, like the per-stage
- * path, and several times faster at T = 1). x and the routing travel through
- * the pinned staging buffer with queued copies, so the call waits for the
- * device once (in the status read). Returns 1 (x untouched) when the launch
+ * path, and several times faster at T = 1). x, the routing and the status
+ * travel through the pinned staging buffer, so the call waits for the device
+ * once. Returns 1 (x untouched) when the launch
  * aborted: the caller then runs the layer per stage. */
 static int decode_one_layer(mia_moe *m, int layer, float *x, const float *bias, int *idx,
                             float *w) {
     const size_t d = (size_t)m->dims.dim, E = (size_t)m->dims.n_experts,
                  K = (size_t)m->dims.n_active;
-    float *hx = m->h_stage, *hy = m->h_stage + d, *hw = m->h_stage + 2 * d + K;
-    int *hi = (int *)(m->h_stage + 2 * d);
+    float *hx = m->h_stage, *hy = m->h_stage + d;
     if (layer < 0 || layer >= m->n_layers) return fail(m, "layer %d out of range", layer);
     memcpy(hx, x, d * 4);
-    if (mhip_h2d_async(m->gpu, m->d_x, hx, d * 4)) return gpu_fail(m);
+    if (mhip_decode_in(m->gpu, m->d_x, hx, (int)d)) return gpu_fail(m);
     if (bias && mhip_h2d(m->gpu, m->d_bias, bias, E * 4)) return gpu_fail(m);
     if (mhip_decode_stack(m->gpu, &m->dims, &m->lay,
                           (const unsigned char *)m->d_table +
@@ -401,17 +410,14 @@ static int decode_one_layer(mia_moe *m, int layer, float *x, const float *bias, 
                           m->d_didx + layer * K, m->d_dw + layer * K,
                           m->flags | MHIP_FORCE_EXACT_ROUTER))
         return gpu_fail(m);
-    if (mhip_d2h_async(m->gpu, hy, m->d_x, d * 4) ||
-        mhip_d2h_async(m->gpu, hi, m->d_didx + layer * K, K * 4) ||
-        mhip_d2h_async(m->gpu, hw, m->d_dw + layer * K, K * 4))
-        return gpu_fail(m);
     int st[4];
-    /* the status read waits for the stream, copies above included */
-    if (mhip_decode_status(m->gpu, m->d_dws, st)) return gpu_fail(m);
+    if (mhip_decode_out(m->gpu, m->d_dws, m->d_x, (int)d, m->d_didx + layer * K,
+                        m->d_dw + layer * K, (int)K, hy, st))
+        return gpu_fail(m);
     if (st[0]) return 1;
     memcpy(x, hy, d * 4);
-    if (idx) memcpy(idx, hi, K * 4);
-    if (w) memcpy(w, hw, K * 4);
+    if (idx) memcpy(idx, hy + d, K * 4);
+    if (w) memcpy(w, hy + d + K, K * 4);
     return 0;
 }
 
