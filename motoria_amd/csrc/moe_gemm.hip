@@ -22,11 +22,18 @@
 // reads Q8(xn); no operand is ever rounded to fp16.
 //
 // Tiles: 256 weight rows x 128 assignments (rows of one expert's bucket),
-// one 32-value Q8_0 block of k per step. Wavefront w owns weight rows
-// 64w..64w+63 against all 128 assignments: 4 x 8 tiles of 16x16 with the
-// weights as the A operand, so each lane's four results share one
-// assignment (one x scale) and four consecutive weight rows (one float4 of
-// weight scales). Two gate/up or three down workgroups share a CU.
+// one 32-value Q8_0 block of k per step, eight wavefronts and two workgroups
+// per CU. The weights are the A operand, so each lane's four results share
+// one assignment (one x scale) and four consecutive weight rows (one float4
+// of weight scales). A tile of more than 64 rows gives a wavefront 64 weight
+// rows against one half of the assignments (4 x 4 tiles of 16 x 16), a tile
+// of fewer 32 weight rows against all of them (2 x up to 4), so that both
+// keep every wavefront busy on at most 64 accumulator registers: four
+// wavefronts per SIMD, of which a vector operation of one runs beside another
+// wavefront's (one alone issues one every ~4.3 cycles, several together one
+// every ~2.1). Against four wavefronts of 64 weight rows x 128 assignments
+// (two per SIMD), same-box: gate/up + down 151 + 80 -> 133 + 75 us at T =
+// 512; the layer 598 -> 572 at T = 2048 skewed, 914 -> 905 at T = 4096.
 //
 // Operands move from global memory straight into an NS-stage LDS ring with
 // global_load_lds (no registers on the way), NS-1 steps ahead of the
@@ -44,18 +51,18 @@ typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef float f4v __attribute__((ext_vector_type(4)));
 
-constexpr int GT = 256;           // threads per workgroup (4 wavefronts)
+constexpr int GT = 512;           // threads per workgroup (8 wavefronts)
 constexpr int TM = MHIP_GEMM_TM;  // assignment rows per tile
 constexpr int TN = 256;           // weight rows per tile
 constexpr int KB = 32;            // k per step: one Q8_0 block
-constexpr int WN = TN / 4;        // weight rows per wavefront (64)
-constexpr int MI = WN / 16;       // 16-row weight tiles per wavefront (4)
-constexpr int NJ = TM / 16;       // 16-row assignment tiles (8)
+constexpr int WN = TN / 4;        // weight rows of a heavy tile's wavefront (64)
+constexpr int MI = WN / 16;       // its 16-row weight tiles (4)
+constexpr int NJ = TM / 32;       // its 16-row assignment tiles (4)
 constexpr int NS = 4;             // ring stages (two workgroups per CU)
 constexpr int OLD = TM + 4;       // gate/up epilogue tile row stride (floats): 128 columns + pad
-constexpr int DLD = WN + 4;       // down epilogue tile row stride: 64 columns + pad
+constexpr int DLD = TN / 2 + 4;   // down epilogue tile row stride: 128 columns + pad
 
-static_assert(TM == 128 && TN == 256 && GT == 256, "tiling");
+static_assert(TM == 128 && TN == 256 && GT == 512, "tiling");
 
 // One step of the ring.
 //   x:  assignment rows, 32 fp16 codes = 4 chunks of 16 bytes; chunk c
@@ -181,69 +188,139 @@ __device__ __forceinline__ h8 codes8(unsigned w0, unsigned w1) {
     return r;
 }
 
-// Per-thread global sources of one tile, advanced by one block per step.
+// Per-thread global sources of one tile, advanced by one block per step:
+// every wavefront copies 16 assignment rows, 32 weight rows and 64 scales
+// (wavefronts 0-3 the weight rows', 4 and 5 the assignment rows', 6 and 7
+// those again).
 struct Src {
-    const _Float16 *x0, *x1;  // assignment-row chunks (KB halves per step)
-    const int8_t *w0, *w1;    // weight-row halves (KB bytes per step)
-    const float *sw;          // this lane's weight-row scale, block-major ...
-    int swstep;               // ... blocks swstep floats apart
-    const float *sx;          // this lane's assignment-row scale (lanes < 32)
-    int sxstep;
+    const _Float16 *x;  // assignment-row chunk (KB halves per step)
+    const int8_t *w;    // weight-row half (KB bytes per step)
+    const float *s;     // scale, block-major ...
+    int sstep;          // ... blocks sstep floats apart
 };
 
-// This thread's four 16-byte pieces of a step: x rows 32 w + lane / 4 and
-// 32 w + 16 + lane / 4 (the chunk that lands in slot lane % 4), weight rows
-// 64 w + lane / 2 and 64 w + 32 + lane / 2 (the half that lands in slot
-// lane % 2).
+// This thread's 16-byte pieces of a step: x row 16 w + lane / 4 (the chunk
+// that lands in slot lane % 4), weight row 32 w + lane / 2 (the half that
+// lands in slot lane % 2); the place of its scale among sx.
 struct Pieces {
-    int xr0, xc0, xr1, xc1, wr0, wh0, wr1, wh1;
+    int xr, xc, wr, wh, sx;
 };
 __device__ __forceinline__ Pieces pieces() {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     Pieces p;
-    p.xr0 = 32 * wave + (lane >> 2);
-    p.xr1 = p.xr0 + 16;
-    p.xc0 = xslot(p.xr0, lane & 3);  // slot ^ swizzle = the chunk stored there
-    p.xc1 = xslot(p.xr1, lane & 3);
-    p.wr0 = 64 * wave + (lane >> 1);
-    p.wr1 = p.wr0 + 32;
-    p.wh0 = wslot(p.wr0, lane & 1);
-    p.wh1 = wslot(p.wr1, lane & 1);
+    p.xr = 16 * wave + (lane >> 2);
+    p.xc = xslot(p.xr, lane & 3);  // slot ^ swizzle = the chunk stored there
+    p.wr = 32 * wave + (lane >> 1);
+    p.wh = wslot(p.wr, lane & 1);
+    p.sx = 64 * (wave & 1) + lane;
     return p;
 }
 
-// The k loop over nk steps (nk >= NS - 1). On return acc[i][j][r] holds
-//   C[64*wave + 16*i + 4*(lane/16) + r][16*j + lane%16]
-// (weight row, assignment row) for the assignment tiles j < NJA (the tiles
-// that hold rows of the bucket; the others are not computed): the exact
-// block dots, each block term added with its two scales in block order.
+// This lane's places in a step, in bytes from its start, at the wavefront's
+// first tiles: tiles are whole 16-row groups, and a row's slots depend on the
+// low bits of its index alone, so the other tiles lie at fixed distances.
+struct Lanes {
+    unsigned x, w, sw, sx;
+};
+
+// One step's products and terms of a wavefront: MIA 16-row weight tiles,
+// nstep rows apart, against NJA assignment tiles.
+template <bool EXACT, int MIA, int NJA>
+__device__ __forceinline__ void step(const char *S, const Lanes &la, int nstep,
+                                     f4v (&acc)[MI * NJ]) {
+    const f4v z = {0.0f, 0.0f, 0.0f, 0.0f};
+    h8 x[NJA];
+#pragma unroll
+    for (int j = 0; j < NJA; j++) x[j] = *(const h8 *)(S + la.x + j * 16 * KB * 2);
+    const f4v sx = *(const f4v *)(S + la.sx);
+    uint2 q = *(const uint2 *)(S + la.w);
+    f4v sw = *(const f4v *)(S + la.sw);
+#pragma unroll
+    for (int i = 0; i < MIA; i++) {
+        const h8 a = codes8(q.x, q.y);
+        f4v blk[NJA];
+#pragma unroll
+        for (int j = 0; j < NJA; j++)
+            blk[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, x[j], z, 0, 0, 0);
+        const f4v s4 = sw;
+        if (i + 1 < MIA) {
+            q = *(const uint2 *)(S + la.w + (i + 1) * nstep * KB);
+            sw = *(const f4v *)(S + la.sw + (i + 1) * nstep * 4);
+        }
+#pragma unroll
+        for (int j = 0; j < NJA; j++) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float t = blk[j][r] * s4[r];
+                if (EXACT)
+                    acc[i * NJ + j][r] = acc[i * NJ + j][r] + t * sx[j];  // no contraction (-ffp-contract=off)
+                else
+                    acc[i * NJ + j][r] = __builtin_fmaf(t, sx[j], acc[i * NJ + j][r]);
+            }
+            // the next tile's products start after this one's terms: started
+            // all at once they would hold 64 registers
+            asm volatile("" : "+v"(acc[i * NJ + j]), "+v"(q.x), "+v"(q.y));
+        }
+    }
+}
+
+// A wavefront's place in a tile. A heavy tile (over TM / 2 rows): weight rows
+// 64 (w % 4) .. + 63, the assignment rows' half w / 4. A light one: 32 weight
+// rows against all its rows.
+struct Place {
+    bool heavy;
+    int n0, j0, nj;  // LDS weight row of its first tile; assignment tiles j0 .. + nj
+};
+__device__ __forceinline__ Place place_of(int nrows, int wave, bool paired) {
+    Place p;
+    p.heavy = nrows > TM / 2;
+    if (p.heavy) {
+        p.n0 = WN * (wave & 3);
+        p.j0 = NJ * (wave >> 2);
+        p.nj = min(NJ, (nrows + 15) / 16 - p.j0);
+    } else {
+        // gate/up pairs a gate tile with the up tile 32 rows on
+        p.n0 = paired ? WN * (wave >> 1) + 16 * (wave & 1) : 32 * wave;
+        p.j0 = 0;
+        p.nj = (nrows + 15) / 16;
+    }
+    return p;
+}
+
+// The k loop over nk steps (nk >= NS - 1). On return acc[NJ i + j][r] holds
+//   C[n0 + 16 i + 4 (lane / 16) + r][16 (j0 + j) + lane % 16]
+// (weight row, assignment row; a light tile's second weight tile lies NSTEP
+// rows on) for j < nj: the exact block dots, each block
+// term added with its two scales in block order.
 // EXACT: the reference's three roundings, s = s + ((float)acc * d_w) * d_x
 // (bit-equal row sums); otherwise the second product and the addition are
 // one fused multiply-add (within a few ulps).
-template <bool EXACT, int NJA>
-__device__ __forceinline__ void gemm_tile(Step *ring, const Src &src, int nk, f4v acc[MI][NJ]) {
-    static_assert(NJA >= 1 && NJA <= NJ, "assignment tiles");
+template <bool EXACT, int MIA, int NJA, int NSTEP>
+__device__ __forceinline__ void gemm_tile(Step *ring, const Src &src, int nk, const Place &pl,
+                                          f4v (&acc)[MI * NJ]) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    constexpr int NLOAD = 6;  // global_load_lds per wavefront per step
+    constexpr int NLOAD = 3;  // global_load_lds per wavefront per step
     const unsigned ring0 = lds_addr(ring);
-    const unsigned ox = (unsigned)offsetof(Step, x) + (2 * wave) * 1024;
-    const unsigned ow = (unsigned)offsetof(Step, w) + (2 * wave) * 1024;
-    const unsigned osw = (unsigned)offsetof(Step, sw) + wave * 256;
-    const unsigned osx = (unsigned)offsetof(Step, sx) + wave * 128;
+    const unsigned ox = (unsigned)offsetof(Step, x) + wave * 1024;
+    const unsigned ow = (unsigned)offsetof(Step, w) + wave * 1024;
+    const unsigned os = wave < 4 ? (unsigned)offsetof(Step, sw) + wave * 256
+                                 : (unsigned)offsetof(Step, sx) + (wave & 1) * 256;
     auto issue = [&](int kb) {
         const int k = min(kb, nk - 1);  // past the end: reload the last step
         const unsigned st = ring0 + (unsigned)((kb % NS) * sizeof(Step));
-        dma16(st + ox, src.x0 + (size_t)k * KB);
-        dma16(st + ox + 1024, src.x1 + (size_t)k * KB);
-        dma16(st + ow, src.w0 + (size_t)k * KB);
-        dma16(st + ow + 1024, src.w1 + (size_t)k * KB);
-        dma4(st + osw, src.sw + (size_t)k * src.swstep);
-        if (lane < 32) dma4(st + osx, src.sx + (size_t)k * src.sxstep);
+        dma16(st + ox, src.x + (size_t)k * KB);
+        dma16(st + ow, src.w + (size_t)k * KB);
+        dma4(st + os, src.s + (size_t)k * src.sstep);
     };
 #pragma unroll
     for (int s = 0; s < NS - 1; s++) issue(s);
     const int c = lane >> 4, l16 = lane & 15;
+    Lanes la;
+    la.x = (unsigned)offsetof(Step, x) + (16 * pl.j0 + l16) * KB * 2 + 16 * xslot(l16, c);
+    la.w = (unsigned)offsetof(Step, w) + (pl.n0 + l16) * KB + 16 * wslot(l16, c >> 1) + 8 * (c & 1);
+    la.sw = (unsigned)offsetof(Step, sw) + (pl.n0 + 4 * c) * 4;
+    la.sx = (unsigned)offsetof(Step, sx) + (8 * l16 + pl.j0) * 4;
     for (int kb = 0; kb < nk; kb++) {
         // this wavefront's loads of step kb are done (NS - 2 later steps may
         // still be in flight); then every wavefront's are
@@ -253,74 +330,33 @@ __device__ __forceinline__ void gemm_tile(Step *ring, const Src &src, int nk, f4
         // wavefront has finished with (the LDS reads completed before the
         // barrier)
         issue(kb + NS - 1);
-        const Step &S = ring[kb % NS];
-        h8 av[MI];
-        f4v s4[MI];
-#pragma unroll
-        for (int i = 0; i < MI; i++) {
-            // weight row n, codes 8c .. 8c+7
-            const int n = WN * wave + 16 * i + l16;
-            const uint2 q = *(const uint2 *)&S.w[n][16 * wslot(n, c >> 1) + 8 * (c & 1)];
-            av[i] = codes8(q.x, q.y);
-            s4[i] = *(const f4v *)&S.sw[WN * wave + 16 * i + 4 * c];
-        }
-        // The block dots of assignment tile j + 1 are started before the
-        // terms of tile j are added, so the vector ALUs never wait for the
-        // product they consume.
-        const f4v z = {0.0f, 0.0f, 0.0f, 0.0f};
-        // x scales of this lane's assignment rows 16 j + l16, j < 8
-        const f4v sxa = *(const f4v *)&S.sx[8 * l16], sxb = *(const f4v *)&S.sx[8 * l16 + 4];
-        f4v blk[2][MI];
-        {
-            const h8 bv = *(const h8 *)&S.x[l16][8 * xslot(l16, c)];
-#pragma unroll
-            for (int i = 0; i < MI; i++)
-                blk[0][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[i], bv, z, 0, 0, 0);
-        }
-#pragma unroll
-        for (int j = 0; j < NJA; j++) {
-            if (j + 1 < NJA) {
-                const int m1 = 16 * (j + 1) + l16;
-                const h8 bv = *(const h8 *)&S.x[m1][8 * xslot(m1, c)];
-#pragma unroll
-                for (int i = 0; i < MI; i++)
-                    blk[(j + 1) & 1][i] =
-                        __builtin_amdgcn_mfma_f32_16x16x32_f16(av[i], bv, z, 0, 0, 0);
-            }
-            const float sx = j < 4 ? sxa[j & 3] : sxb[j & 3];
-#pragma unroll
-            for (int i = 0; i < MI; i++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const float t = blk[j & 1][i][r] * s4[i][r];
-                    if (EXACT)
-                        acc[i][j][r] = acc[i][j][r] + t * sx;  // no contraction (-ffp-contract=off)
-                    else
-                        acc[i][j][r] = __builtin_fmaf(t, sx, acc[i][j][r]);
-                }
-        }
+        step<EXACT, MIA, NJA>((const char *)&ring[kb % NS], la, NSTEP, acc);
     }
     wait_vm<0>();  // the reloads past the end
     __syncthreads();
 }
 
-// The assignment tiles that hold rows of the bucket (a bucket's last tile
-// may hold few rows).
-template <bool EXACT>
-__device__ __forceinline__ void gemm_tile_rows(Step *ring, const Src &src, int nk, int nrows,
-                                               f4v acc[MI][NJ]) {
-    // one instantiation per count of 16-row tiles, so a bucket's last tile
-    // runs no empty tile (gate/up 468 -> 459 us at T = 4096, 157 -> 149 us
-    // at T = 512, against rounding the count up to a power of two)
-    switch ((nrows + 15) / 16) {
-    case 8: gemm_tile<EXACT, 8>(ring, src, nk, acc); break;
-    case 7: gemm_tile<EXACT, 7>(ring, src, nk, acc); break;
-    case 6: gemm_tile<EXACT, 6>(ring, src, nk, acc); break;
-    case 5: gemm_tile<EXACT, 5>(ring, src, nk, acc); break;
-    case 4: gemm_tile<EXACT, 4>(ring, src, nk, acc); break;
-    case 3: gemm_tile<EXACT, 3>(ring, src, nk, acc); break;
-    case 2: gemm_tile<EXACT, 2>(ring, src, nk, acc); break;
-    default: gemm_tile<EXACT, 1>(ring, src, nk, acc); break;
+// The k loop in the form of the wavefront's place: one per count of 16-row
+// assignment tiles, so a bucket's last tile runs no empty tile. (The two
+// halves of a heavy tile may take different forms: the choice is a
+// wavefront's, and every form meets nk + 1 barriers.)
+template <bool EXACT, int NSTEP>
+__device__ __forceinline__ void gemm_tile_rows(Step *ring, const Src &src, int nk, const Place &pl,
+                                               f4v (&acc)[MI * NJ]) {
+    if (pl.heavy) {
+        switch (pl.nj) {
+        case 4: gemm_tile<EXACT, MI, 4, 16>(ring, src, nk, pl, acc); break;
+        case 3: gemm_tile<EXACT, MI, 3, 16>(ring, src, nk, pl, acc); break;
+        case 2: gemm_tile<EXACT, MI, 2, 16>(ring, src, nk, pl, acc); break;
+        default: gemm_tile<EXACT, MI, 1, 16>(ring, src, nk, pl, acc); break;
+        }
+    } else {
+        switch (pl.nj) {
+        case 4: gemm_tile<EXACT, MI / 2, 4, NSTEP>(ring, src, nk, pl, acc); break;
+        case 3: gemm_tile<EXACT, MI / 2, 3, NSTEP>(ring, src, nk, pl, acc); break;
+        case 2: gemm_tile<EXACT, MI / 2, 2, NSTEP>(ring, src, nk, pl, acc); break;
+        default: gemm_tile<EXACT, MI / 2, 1, NSTEP>(ring, src, nk, pl, acc); break;
+        }
     }
 }
 
@@ -362,7 +398,7 @@ union alignas(16) GateUpLds {
 };
 union alignas(16) DownLds {
     Step ring[NS];
-    float o[TM][DLD];  // epilogue: 128 assignment rows x 64 down rows
+    float o[TM][DLD];  // epilogue: 128 assignment rows x 128 down rows
 };
 static_assert(sizeof(GateUpLds) == NS * sizeof(Step) && sizeof(DownLds) == NS * sizeof(Step),
               "epilogue tiles fit the rings");
@@ -374,7 +410,7 @@ static_assert(2 * sizeof(DownLds) <= 160 * 1024, "two workgroups per CU");
 // 128 consecutive h columns h0..h0+127. Wavefront w's 64 weight rows are the
 // gate rows then the up rows of h columns h0+32w..h0+32w+31, so SwiGLU pairs
 // its accumulator tiles i and i + 2 lane by lane.
-__global__ __launch_bounds__(GT, 2) void k_gateup_mfma(
+__global__ __launch_bounds__(GT, 4) void k_gateup_mfma(
     const uint8_t *__restrict__ table, mhip_layout lay, const _Float16 *__restrict__ xq16,
     const float *__restrict__ xsb, const int *__restrict__ groups, const int *__restrict__ gtile,
     const int *__restrict__ glight, const int *__restrict__ perm, _Float16 *__restrict__ hq16,
@@ -392,10 +428,7 @@ __global__ __launch_bounds__(GT, 2) void k_gateup_mfma(
     Src src;
     {
         const Pieces p = pieces();
-        const int t0 = perm[base + min(p.xr0, nrows - 1)] / K;
-        const int t1 = perm[base + min(p.xr1, nrows - 1)] / K;
-        src.x0 = xq16 + (size_t)t0 * d + p.xc0 * 8;
-        src.x1 = xq16 + (size_t)t1 * d + p.xc1 * 8;
+        src.x = xq16 + (size_t)(perm[base + min(p.xr, nrows - 1)] / K) * d + p.xc * 8;
         // tile row n: wavefront n / 64; within it gate rows then up rows
         auto wrow = [&](int n, int half) {
             const int r = n % WN;
@@ -403,77 +436,77 @@ __global__ __launch_bounds__(GT, 2) void k_gateup_mfma(
             return (const int8_t *)(ex + (r < WN / 2 ? lay.gate_q : lay.up_q)) + (size_t)hc * d +
                    16 * half;
         };
-        src.w0 = wrow(p.wr0, p.wh0);
-        src.w1 = wrow(p.wr1, p.wh1);
-        {
+        src.w = wrow(p.wr, p.wh);
+        if (wave < 4) {
             // scale of tile row 64 wave + lane
             const int hc = h0 + wave * (WN / 2) + lane % (WN / 2);
-            src.sw = (const float *)(ex + (lane < WN / 2 ? lay.gate_st : lay.up_st)) + hc;
-            src.swstep = eh;
+            src.s = (const float *)(ex + (lane < WN / 2 ? lay.gate_st : lay.up_st)) + hc;
+            src.sstep = eh;
+        } else {
+            // sx slot p holds bucket row 16 (p % 8) + p / 8
+            src.s = xsb + base + min(16 * (p.sx & 7) + (p.sx >> 3), nrows - 1);
+            src.sstep = A;
         }
-        {
-            // sx slot p = 32 wave + lane holds bucket row 16 (p % 8) + p / 8
-            const int p = 32 * wave + (lane & 31);
-            src.sx = xsb + base + min(16 * (p & 7) + (p >> 3), nrows - 1);
-        }
-        src.sxstep = A;
     }
 
-    f4v acc[MI][NJ];
+    f4v acc[MI * NJ];
 #pragma unroll
-    for (int i = 0; i < MI; i++)
-#pragma unroll
-        for (int j = 0; j < NJ; j++) acc[i][j] = (f4v){0.0f, 0.0f, 0.0f, 0.0f};
-    gemm_tile_rows<true>(L.ring, src, d / KB, nrows, acc);
+    for (int i = 0; i < MI * NJ; i++) acc[i] = (f4v){0.0f, 0.0f, 0.0f, 0.0f};
+    const Place pl = place_of(nrows, __builtin_amdgcn_readfirstlane(wave), true);
+    gemm_tile_rows<true, 32>(L.ring, src, d / KB, pl, acc);
 
     // SwiGLU into the h tile (LDS, reused): row = assignment, column = h - h0
     const int c = lane >> 4, l16 = lane & 15;
+    auto swiglu = [&](const f4v &g, const f4v &u, int row, int col) {
+        f4v hv;
 #pragma unroll
-    for (int i = 0; i < MI / 2; i++)
+        for (int r = 0; r < 4; r++)
+            hv[r] = (g[r] / (1.0f + mia_expf_glibc_tab(-g[r], etab))) * u[r];
+        *(f4v *)&L.o[row][col] = hv;
+    };
 #pragma unroll
-        for (int j = 0; j < NJ; j++) {
-            f4v hv;
+    for (int j = 0; j < NJ; j++) {
+        if (j < pl.nj) {
+            const int row = 16 * (pl.j0 + j) + l16;
+            if (pl.heavy) {
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const float gv = acc[i][j][r], uv = acc[i + 2][j][r];
-                hv[r] = (gv / (1.0f + mia_expf_glibc_tab(-gv, etab))) * uv;
+                for (int i = 0; i < MI / 2; i++)
+                    swiglu(acc[i * NJ + j], acc[(i + 2) * NJ + j], row,
+                           (WN / 2) * (wave & 3) + 16 * i + 4 * c);
+            } else {
+                swiglu(acc[j], acc[NJ + j], row, 16 * wave + 4 * c);
             }
-            *(f4v *)&L.o[16 * j + l16][(WN / 2) * wave + 16 * i + 4 * c] = hv;
         }
+    }
     __syncthreads();
     {
         // Q8_0 of 32-blocks of h (quant.c:11-27): the codes as fp16 integers
         // (bucketed rows) and the scales block-major (hsb[block][row], the
-        // down kernel's x scales); thread (m, b2) does blocks 2 b2 and
-        // 2 b2 + 1 of row m
-        const int m = tid >> 1, b2 = tid & 1;
+        // down kernel's x scales); a thread per (row, block)
+        const int m = tid >> 2, blk = tid & 3;
         if (m < nrows) {
+            const f4v *hs = (const f4v *)&L.o[m][32 * blk];
+            float v[32];
 #pragma unroll
-            for (int bb = 0; bb < 2; bb++) {
-                const int blk = 2 * b2 + bb;
-                const f4v *hs = (const f4v *)&L.o[m][32 * blk];
-                float v[32];
-#pragma unroll
-                for (int k = 0; k < 8; k++) {
-                    const f4v q = hs[k];
-                    v[4 * k] = q[0];
-                    v[4 * k + 1] = q[1];
-                    v[4 * k + 2] = q[2];
-                    v[4 * k + 3] = q[3];
-                }
-                float amax = 0.0f;
-#pragma unroll
-                for (int k = 0; k < 32; k++) amax = fmaxf(amax, fabsf(v[k]));
-                const float dsc = amax / 127.0f;
-                const float qi = dsc != 0.0f ? 1.0f / dsc : 0.0f;
-                h8 o[4];
-#pragma unroll
-                for (int k = 0; k < 32; k++) o[k >> 3][k & 7] = (_Float16)roundf(v[k] * qi);
-                h8 *dst = (h8 *)(hq16 + (size_t)(base + m) * eh + h0 + 32 * blk);
-#pragma unroll
-                for (int k = 0; k < 4; k++) dst[k] = o[k];
-                hsb[(size_t)(h0 / KB + blk) * A + base + m] = dsc;
+            for (int k = 0; k < 8; k++) {
+                const f4v q = hs[k];
+                v[4 * k] = q[0];
+                v[4 * k + 1] = q[1];
+                v[4 * k + 2] = q[2];
+                v[4 * k + 3] = q[3];
             }
+            float amax = 0.0f;
+#pragma unroll
+            for (int k = 0; k < 32; k++) amax = fmaxf(amax, fabsf(v[k]));
+            const float dsc = amax / 127.0f;
+            const float qi = dsc != 0.0f ? 1.0f / dsc : 0.0f;
+            h8 o[4];
+#pragma unroll
+            for (int k = 0; k < 32; k++) o[k >> 3][k & 7] = (_Float16)roundf(v[k] * qi);
+            h8 *dst = (h8 *)(hq16 + (size_t)(base + m) * eh + h0 + 32 * blk);
+#pragma unroll
+            for (int k = 0; k < 4; k++) dst[k] = o[k];
+            hsb[(size_t)(h0 / KB + blk) * A + base + m] = dsc;
         }
     }
 }
@@ -488,7 +521,7 @@ __global__ __launch_bounds__(GT, 2) void k_gateup_mfma(
 // EXACT: the reference's roundings of each block term (the expert outputs
 // bit-equal); otherwise one fused multiply-add per term (a few ulps).
 template <bool EXACT>
-__global__ __launch_bounds__(GT, 2) void k_down_mfma(const uint8_t *__restrict__ table,
+__global__ __launch_bounds__(GT, 4) void k_down_mfma(const uint8_t *__restrict__ table,
                                                      mhip_layout lay,
                                                      const _Float16 *__restrict__ hq16,
                                                      const float *__restrict__ hsb,
@@ -508,44 +541,46 @@ __global__ __launch_bounds__(GT, 2) void k_down_mfma(const uint8_t *__restrict__
     Src src;
     {
         const Pieces p = pieces();
-        src.x0 = hq16 + (size_t)(base + min(p.xr0, nrows - 1)) * eh + p.xc0 * 8;
-        src.x1 = hq16 + (size_t)(base + min(p.xr1, nrows - 1)) * eh + p.xc1 * 8;
-        const int8_t *dq = (const int8_t *)(ex + lay.down_q);
-        src.w0 = dq + (size_t)(n0 + p.wr0) * eh + 16 * p.wh0;
-        src.w1 = dq + (size_t)(n0 + p.wr1) * eh + 16 * p.wh1;
-        src.sw = (const float *)(ex + lay.down_st) + n0 + WN * wave + lane;
-        src.swstep = d;
-        // sx slot p = 32 wave + lane holds bucket row 16 (p % 8) + p / 8
-        const int ps = 32 * wave + (lane & 31);
-        src.sx = hsb + base + min(16 * (ps & 7) + (ps >> 3), nrows - 1);
-        src.sxstep = A;
+        src.x = hq16 + (size_t)(base + min(p.xr, nrows - 1)) * eh + p.xc * 8;
+        src.w = (const int8_t *)(ex + lay.down_q) + (size_t)(n0 + p.wr) * eh + 16 * p.wh;
+        if (wave < 4) {
+            src.s = (const float *)(ex + lay.down_st) + n0 + WN * wave + lane;
+            src.sstep = d;
+        } else {
+            // sx slot p holds bucket row 16 (p % 8) + p / 8
+            src.s = hsb + base + min(16 * (p.sx & 7) + (p.sx >> 3), nrows - 1);
+            src.sstep = A;
+        }
     }
 
-    f4v acc[MI][NJ];
+    f4v acc[MI * NJ];
 #pragma unroll
-    for (int i = 0; i < MI; i++)
-#pragma unroll
-        for (int j = 0; j < NJ; j++) acc[i][j] = (f4v){0.0f, 0.0f, 0.0f, 0.0f};
-    gemm_tile_rows<EXACT>(L.ring, src, eh / KB, nrows, acc);
+    for (int i = 0; i < MI * NJ; i++) acc[i] = (f4v){0.0f, 0.0f, 0.0f, 0.0f};
+    const Place pl = place_of(nrows, __builtin_amdgcn_readfirstlane(wave), false);
+    gemm_tile_rows<EXACT, 16>(L.ring, src, eh / KB, pl, acc);
 
     const int c = lane >> 4, l16 = lane & 15;
 #pragma unroll
-    for (int qw = 0; qw < 4; qw++) {
-        // wavefront qw's 64 columns, then every thread writes them out
-        if (wave == qw) {
+    for (int half = 0; half < 2; half++) {
+        // the tile's columns 128 half .. + 127, then every thread writes them out
+        if (pl.n0 / (TN / 2) == half) {
 #pragma unroll
-            for (int i = 0; i < MI; i++)
+            for (int j = 0; j < NJ; j++)
+                if (j < pl.nj) {
 #pragma unroll
-                for (int j = 0; j < NJ; j++)
-                    *(f4v *)&L.o[16 * j + l16][16 * i + 4 * c] = acc[i][j];
+                    for (int i = 0; i < MI; i++)
+                        if (pl.heavy || i < MI / 2)
+                            *(f4v *)&L.o[16 * (pl.j0 + j) + l16][pl.n0 % (TN / 2) + 16 * i + 4 * c] =
+                                acc[i * NJ + j];
+                }
         }
         __syncthreads();
-        // 128 rows x 16 float4: thread tid writes float4 tid % 16 of rows tid / 16 + 16 k
+        // 128 rows x 32 float4: thread tid writes float4 tid % 32 of rows tid / 32 + 16 k
 #pragma unroll
         for (int k = 0; k < TM / 16; k++) {
-            const int m = tid / 16 + 16 * k, f = tid % 16;
+            const int m = tid / 32 + 16 * k, f = tid % 32;
             if (m < nrows)
-                *(f4v *)(tmp + (size_t)(base + m) * d + n0 + WN * qw + 4 * f) =
+                *(f4v *)(tmp + (size_t)(base + m) * d + n0 + (TN / 2) * half + 4 * f) =
                     *(const f4v *)&L.o[m][4 * f];
         }
         __syncthreads();
