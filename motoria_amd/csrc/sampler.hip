@@ -4,9 +4,10 @@
 //   greedy:  the first maximum (k_argmax_part / k_argmax_final; NaN never
 //            wins except at index 0, as the reference's strict comparison)
 //   else:    e_i = expf((l_i - l_best) / T)            (k_sample_exp)
-//            sum = e_0 + e_1 + ... in index order       (k_chain_sum)
-//            candidates p_i = e_i / sum >= cutoff as 64-bit keys
-//            (descending p, ascending index), sorted    (k_sample_keys, rocPRIM)
+//            sum = e_0 + e_1 + ... in index order       (k_sum_runs, k_sum_walk;
+//                                                        k_chain_sum)
+//            candidates p_i = e_i / sum >= cutoff as keys (descending
+//            p) and indices, sorted stably              (k_sample_keys, rocPRIM)
 //            the running sum of the sorted p up to top_p, r = u * cum, the
 //            first candidate whose running sum exceeds r (k_sample_pick)
 //
@@ -24,7 +25,7 @@ namespace {
 
 constexpr int NT = 256;          // threads of every sampler kernel
 constexpr int PARTS = 256;       // workgroups of the argmax's first pass
-constexpr uint64_t NONE = ~0ull; // key of a dropped token
+constexpr uint32_t NONE = ~0u;    // key of a dropped token
 
 struct SampleState {
     int best;
@@ -90,17 +91,45 @@ __global__ __launch_bounds__(NT) void k_argmax_final(const float *__restrict__ l
     }
 }
 
-// sampler.c:41-44, the exponentials (the sum is k_chain_sum's).
-__global__ __launch_bounds__(NT) void k_sample_exp(const float *__restrict__ l, int n,
-                                                   float temperature,
-                                                   const SampleState *__restrict__ st,
-                                                   float *__restrict__ e) {
+// The sum's pieces (k_sum_runs): a thread takes PIECE consecutive values, 64
+// pieces make a group (a wavefront), RUN_T / 64 groups a workgroup.
+constexpr int RUN_T = 256, PIECE = 8, RUN_W = RUN_T * PIECE;
+// Sizes whose sum is taken so: from where it is faster (a whole draw, us, on
+// one workgroup / so: 4096 95/65, 32768 152/83, 151936 236/131 with spread
+// logits) up to where their groups fit the walk's workgroup, and the
+// workgroups' sums the argmax's partial results.
+constexpr int RUN_MIN_N = 2048, RUN_MAX_N = PARTS * RUN_W;
+
+// sampler.c:41-44, the exponentials (the sum is k_sum_runs' and k_sum_walk's),
+// and (bsum not null) each workgroup's sum of its RUN_W values in double.
+__global__ __launch_bounds__(RUN_T) void k_sample_exp(const float *__restrict__ l, int n,
+                                                      float temperature,
+                                                      const SampleState *__restrict__ st,
+                                                      float *__restrict__ e,
+                                                      double *__restrict__ bsum) {
     __shared__ uint64_t etab[32];
-    if (threadIdx.x < 32) etab[threadIdx.x] = mia_expf_tab[threadIdx.x];
+    __shared__ double part[RUN_T / 64];
+    const int tid = threadIdx.x;
+    if (tid < 32) etab[tid] = mia_expf_tab[tid];
     __syncthreads();
     const float mx = l[st->best];
-    const int i = blockIdx.x * NT + threadIdx.x;
-    if (i < n) e[i] = mia_expf_glibc_tab((l[i] - mx) / temperature, etab);
+    const int i0 = blockIdx.x * RUN_W, i1 = min(n, i0 + RUN_W);
+    double s = 0.0;
+    for (int i = i0 + tid; i < i1; i += RUN_T) {
+        const float v = mia_expf_glibc_tab((l[i] - mx) / temperature, etab);
+        e[i] = v;
+        s = s + (double)v;
+    }
+    if (!bsum) return;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s = s + __shfl_xor(s, o);
+    if ((tid & 63) == 0) part[tid >> 6] = s;
+    __syncthreads();
+    if (tid == 0) {
+        double t = 0.0;
+        for (int k = 0; k < RUN_T / 64; k++) t = t + part[k];
+        bsum[blockIdx.x] = t;
+    }
 }
 
 // ---- exact running sums, 8192 additions at a time -------------------------------
@@ -349,40 +378,228 @@ __global__ __launch_bounds__(SQ_T) void k_chain_sum(const float *__restrict__ e,
     if (threadIdx.x == 0) st->sum = s;
 }
 
+// ---- the same over the whole chip ---------------------------------------------------
+//
+// A run of additions s <- fl(s + v), v >= 0, that stays inside one binade of
+// s is a map of s's bits that depends on their lowest one alone (s = M u;
+// fl(s + v) = (M + k) u, k the integer nearest v / u, a tie to the even M +
+// k), and such maps compose. A double scan of the workgroups' sums tells in
+// which binade nearly every piece will lie. k_sum_runs (all CUs) makes each
+// such piece a map and composes the maps of every 64 pieces between the
+// others, whose places it notes (the first, and those within 2^-14 of a power
+// of two). k_sum_walk, one workgroup, composes what is left over the groups
+// and then goes from one noted piece to the next: a map, the piece's own
+// additions. The scan only predicts (the fp32 sum drifts from the exact one
+// by its roundings); the walk checks each map before it counts: s lies in the
+// binade the map was made for, and still does after it, so, the additions
+// being of values >= 0, it did all along. Where that fails, or with more
+// than WALK_MAX noted pieces (NaN or infinite values, sums among the
+// subnormals), seq_scan runs over all values instead. 151936 values: 108 us
+// for seq_scan on one workgroup, 4 + 8 us for the two; about one in twenty
+// of a model's logits at T = 0.6-1 still needs seq_scan (many values too small
+// to be added move a power of two past its noted pieces).
+struct Run {
+    int a0, a1;  // added to even (odd) bits
+    int P;       // the exponent field of the binade; 0: nothing is added
+};
+__device__ __forceinline__ Run then(Run a, Run b) {
+    return {a.a0 + ((a.a0 & 1) ? b.a1 : b.a0), a.a1 + ((a.a1 & 1) ? b.a0 : b.a1), b.P ? b.P : a.P};
+}
+__device__ __forceinline__ Run run_up(Run r, int o) {
+    return {__shfl_up(r.a0, o), __shfl_up(r.a1, o), __shfl_up(r.P, o)};
+}
+// The runs of the lanes before and this one's, from the last lane with `head`
+// set on (its own included); head: whether there was one.
+__device__ __forceinline__ void wave_runs(Run &r, int &head, int lane) {
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const Run p = run_up(r, o);
+        const int ph = __shfl_up(head, o);
+        if (lane >= o && !head) {
+            r = then(p, r);
+            head = ph;
+        }
+    }
+}
+
+// run[k]: the maps of piece k and those before it in its group, from the last
+// noted piece on (which has none of its own); noted[group]: a bit per piece.
+__global__ __launch_bounds__(RUN_T) void k_sum_runs(const float *__restrict__ e, int n,
+                                                    const double *__restrict__ bsum,
+                                                    Run *__restrict__ run,
+                                                    unsigned long long *__restrict__ noted) {
+    __shared__ double part[RUN_T / 64], before[RUN_T / 64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    double b = 0.0;
+    for (int k = tid; k < (int)blockIdx.x; k += RUN_T) b = b + bsum[k];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) b = b + __shfl_xor(b, o);
+    if (lane == 0) before[wave] = b;
+    const int p = blockIdx.x * RUN_T + tid, i0 = p * PIECE;
+    float v[PIECE];
+#pragma unroll
+    for (int j = 0; j < PIECE; j += 4) {
+        const float4 q = i0 + j < n ? *(const float4 *)(e + i0 + j) : make_float4(0, 0, 0, 0);
+        v[j] = q.x;
+        v[j + 1] = i0 + j + 1 < n ? q.y : 0.0f;
+        v[j + 2] = i0 + j + 2 < n ? q.z : 0.0f;
+        v[j + 3] = i0 + j + 3 < n ? q.w : 0.0f;
+    }
+    double own = 0.0;
+#pragma unroll
+    for (int j = 0; j < PIECE; j++) own = own + (double)v[j];
+    double incl = own;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const double y = __shfl_up(incl, o);
+        if (lane >= o) incl = incl + y;
+    }
+    if (lane == 63) part[wave] = incl;
+    __syncthreads();
+    double base = 0.0;
+    for (int k = 0; k < RUN_T / 64; k++) base = base + before[k];
+    for (int k = 0; k < wave; k++) base = base + part[k];
+    const double S1 = base + incl, S0 = S1 - own, dl = 0x1p-14;
+    const unsigned b0 = (unsigned)((uint64_t)__double_as_longlong(S0 * (1.0 - dl)) >> 52);
+    const unsigned b1 = (unsigned)((uint64_t)__double_as_longlong(S1 * (1.0 + dl)) >> 52);
+    const bool zero = own == 0.0;  // (every value is +0, or past the end)
+    const bool in = zero || (b0 == b1 && b0 >= 1023 - 100 && b0 < 1023 + 100);
+    Run r = {0, 0, 0};
+    if (in && !zero) {
+        // v / u, u = 2^(P - 23), P = b0 - 1023: exact, or too small to count
+        const float scale = __int_as_float((int)(127 + 23 + 1023 - b0) << 23);
+        r.P = (int)b0 - 1023 + 127;
+#pragma unroll
+        for (int j = 0; j < PIECE; j++) {
+            const float q = v[j] * scale, f = floorf(q), fr = q - f;
+            const int k = (int)f, up = fr > 0.5f ? 1 : 0;
+            const bool tie = fr == 0.5f;
+            r.a0 = r.a0 + k + (tie ? (r.a0 + k) & 1 : up);
+            r.a1 = r.a1 + k + (tie ? (r.a1 + k + 1) & 1 : up);
+        }
+    }
+    const unsigned long long mask = __ballot(!in);
+    int head = in ? 0 : 1;
+    wave_runs(r, head, lane);
+    run[p] = r;
+    if (lane == 0) noted[p >> 6] = mask;
+}
+
+constexpr int WALK_MAX = 128;  // noted pieces of the walk, at most
+static_assert(RUN_MAX_N / (64 * PIECE) <= SQ_T, "a thread per group");
+__global__ __launch_bounds__(SQ_T) void k_sum_walk(const float *__restrict__ e, int n, int groups,
+                                                   const Run *__restrict__ run,
+                                                   const unsigned long long *__restrict__ noted,
+                                                   SampleState *st) {
+    __shared__ Run pre[WALK_MAX + 1], wlast[SQ_T / 64];
+    __shared__ int piece[WALK_MAX], whead[SQ_T / 64], wcnt[SQ_T / 64], bad;
+    __shared__ float vals[WALK_MAX][PIECE];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const unsigned long long mask = tid < groups ? noted[tid] : 0;
+    Run r = {0, 0, 0};
+    if (tid < groups) r = run[64 * tid + 63];
+    // runs over the groups, from the last noted piece on, and the count of
+    // noted pieces before each group
+    int head = mask ? 1 : 0, cnt = __popcll(mask);
+    wave_runs(r, head, lane);
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(cnt, o);
+        if (lane >= o) cnt = cnt + y;
+    }
+    if (lane == 63) {
+        wlast[wave] = r;
+        whead[wave] = head;
+        wcnt[wave] = cnt;
+    }
+    if (tid == 0) bad = 0;
+    __syncthreads();
+    Run wb = {0, 0, 0};  // the wavefronts before this one
+    int c0 = 0, total = 0;
+    for (int k = 0; k < SQ_T / 64; k++) {
+        if (k < wave) {
+            wb = whead[k] ? wlast[k] : then(wb, wlast[k]);
+            c0 = c0 + wcnt[k];
+        }
+        total = total + wcnt[k];
+    }
+    if (total <= WALK_MAX) {  // (uniform)
+        const Run incl = head ? r : then(wb, r), up = run_up(incl, 1);
+        const Run before = lane > 0 ? up : wb;  // from the last noted piece up to this group
+        if (tid == SQ_T - 1) pre[total] = incl;
+        int k = c0 + cnt - __popcll(mask), prev = -1;
+        for (unsigned long long left = mask; left; left &= left - 1, k++) {
+            const int i = __ffsll((long long)left) - 1;
+            // the pieces between the noted one before (or the group's start)
+            // and this one: piece i - 1's run starts there
+            Run g = {0, 0, 0};
+            if (i - 1 > prev) g = run[64 * tid + i - 1];
+            pre[k] = prev < 0 ? then(before, g) : g;
+            piece[k] = 64 * tid + i;
+            prev = i;
+        }
+        __syncthreads();
+        for (int q = tid; q < total * PIECE; q += SQ_T) {
+            const int i = piece[q / PIECE] * PIECE + q % PIECE;
+            vals[q / PIECE][q % PIECE] = i < n ? e[i] : 0.0f;
+        }
+        __syncthreads();
+        if (wave == 0) {
+            float s = 0.0f;
+            bool ok = true;
+            for (int q = 0; q <= total; q++) {
+                const Run g = pre[q];
+                const int b = __float_as_int(s), a = (b & 1) ? g.a1 : g.a0;
+                ok = ok && (g.P == 0 || (b >> 23 == g.P && (b + a) >> 23 == g.P));
+                s = __int_as_float(b + a);
+                if (q < total) {
+#pragma unroll
+                    for (int j = 0; j < PIECE; j++) s = s + vals[q][j];
+                }
+            }
+            if (tid == 0) {
+                st->sum = s;
+                bad = !ok;
+            }
+        }
+        __syncthreads();
+        if (!bad) return;
+    }
+    float s;
+    seq_scan<SQ_SUM>(e, n, 0.0f, &s);
+    if (tid == 0) st->sum = s;
+}
+
 // sampler.c:46-51: p_i = e_i / sum; a candidate when p_i >= cutoff, as the
-// key (0x7fffffff - bits(p)) << 32 | i: ascending keys are descending p, and
-// ascending index among equal p (bits of p >= 0 order as p does).
+// key 0x7fffffff - bits(p) with i beside it: ascending keys are descending p
+// (bits of p >= 0 order as p does), and the sort keeps equal ones in index
+// order. (Half the passes of a sort by key and index together: 60 -> 35 us
+// at 151936 values.)
 __global__ __launch_bounds__(NT) void k_sample_keys(const float *__restrict__ e, int n,
                                                     float cutoff,
                                                     const SampleState *__restrict__ st,
-                                                    uint64_t *__restrict__ keys) {
+                                                    uint32_t *__restrict__ keys,
+                                                    int *__restrict__ ids) {
     const int i = blockIdx.x * NT + threadIdx.x;
     if (i >= n) return;
     const float p = e[i] / st->sum;
-    keys[i] = p >= cutoff
-                  ? ((uint64_t)(0x7fffffffu - __float_as_uint(p)) << 32) | (uint32_t)i
-                  : NONE;
+    keys[i] = p >= cutoff ? 0x7fffffffu - __float_as_uint(p) : NONE;
+    ids[i] = i;
 }
 
-__device__ __forceinline__ float key_p(uint64_t k) {
-    return __uint_as_float(0x7fffffffu - (uint32_t)(k >> 32));
-}
-
-// The sorted keys as probabilities pf[] and token ids pi[]; the candidates
-// are the keys before the first NONE: their count goes to st->last (as
-// m - 1, the default last candidate).
-__global__ __launch_bounds__(NT) void k_keys_split(const uint64_t *__restrict__ keys, int n,
-                                                   float *__restrict__ pf, int *__restrict__ pi,
-                                                   SampleState *st) {
+// The sorted keys as probabilities pf[]; the candidates are the keys before
+// the first NONE: their count goes to st->last (as m - 1, the default last
+// candidate).
+__global__ __launch_bounds__(NT) void k_keys_split(const uint32_t *__restrict__ keys, int n,
+                                                   float *__restrict__ pf, SampleState *st) {
     const int i = blockIdx.x * NT + threadIdx.x;
     if (i >= n) return;
-    const uint64_t k = keys[i];
+    const uint32_t k = keys[i];
     if (k == NONE) {
         if (i == 0) st->last = -1;
         return;
     }
-    pf[i] = key_p(k);
-    pi[i] = (int)(uint32_t)k;
+    pf[i] = __uint_as_float(0x7fffffffu - k);
     if (i + 1 == n || keys[i + 1] == NONE) st->last = i;
 }
 
@@ -426,7 +643,7 @@ size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
 // The LDS ring of the running-sum kernels is above the default limit.
 int sq_lds_attr(mhip_ctx *c) {
-    const void *fns[] = {(const void *)k_chain_sum, (const void *)k_sample_pick,
+    const void *fns[] = {(const void *)k_chain_sum, (const void *)k_sum_walk, (const void *)k_sample_pick,
                          (const void *)k_chain<SQ_SUM>, (const void *)k_chain<SQ_GE>,
                          (const void *)k_chain<SQ_GT>};
     for (const void *f : fns)
@@ -442,14 +659,18 @@ struct SampleScratch {
     Best *part;
     float *e;
     uint64_t *kin, *kout;
+    // of the sum, in the places of what is dead or not yet there
+    double *bsum;               // [workgroups of k_sum_runs]: the argmax's partial results
+    Run *run;                   // [pieces]: the first keys
+    unsigned long long *noted;  // [groups]: the sorted keys
     void *tmp;
     size_t tmp_bytes;
 };
 
 size_t sort_bytes(int n) {
     size_t b = 0;
-    if (rocprim::radix_sort_keys(nullptr, b, (const uint64_t *)nullptr, (uint64_t *)nullptr,
-                                 (unsigned)n, 0, 64) != hipSuccess)
+    if (rocprim::radix_sort_pairs(nullptr, b, (const uint32_t *)nullptr, (uint32_t *)nullptr,
+                                  (const int *)nullptr, (int *)nullptr, (unsigned)n, 0, 32) != hipSuccess)
         return 0;
     return b;
 }
@@ -467,6 +688,12 @@ SampleScratch carve(int n, void *base) {
     p += align256((size_t)n * 8);
     s.kout = (uint64_t *)p;
     p += align256((size_t)n * 8);
+    s.bsum = (double *)s.part;
+    s.run = (Run *)s.kin;
+    s.noted = (unsigned long long *)s.kout;
+    static_assert(sizeof(Best) >= sizeof(double), "a sum per partial result");
+    static_assert((RUN_MIN_N + RUN_W) / PIECE * sizeof(Run) <= RUN_MIN_N * sizeof(uint64_t),
+                  "whole workgroups of runs fit the keys");
     s.tmp = p;
     s.tmp_bytes = sort_bytes(n);
     return s;
@@ -521,18 +748,27 @@ int mhip_sample(mhip_ctx *c, mhip_sampler *s, const float *d_logits, void *d_scr
     const float u = rand01(s);
     const float cutoff = (1.0f - s->top_p) / (float)(n > 1 ? n - 1 : 1);
     const unsigned nb = mhip::blocks_for(n, NT);
-    k_sample_exp<<<nb, NT, 0, st>>>(d_logits, n, s->temperature, sc.st, sc.e);
+    const unsigned rb = mhip::blocks_for(n, RUN_W);
+    const bool runs = n >= RUN_MIN_N && n <= RUN_MAX_N;
+    k_sample_exp<<<rb, RUN_T, 0, st>>>(d_logits, n, s->temperature, sc.st, sc.e,
+                                       runs ? sc.bsum : nullptr);
     if (sq_lds_attr(c)) return -1;
-    k_chain_sum<<<1, SQ_T, SQ_LDS, st>>>(sc.e, n, sc.st);
-    k_sample_keys<<<nb, NT, 0, st>>>(sc.e, n, cutoff, sc.st, sc.kin);
+    if (runs) {
+        k_sum_runs<<<rb, RUN_T, 0, st>>>(sc.e, n, sc.bsum, sc.run, sc.noted);
+        k_sum_walk<<<1, SQ_T, SQ_LDS, st>>>(sc.e, n, (int)rb * (RUN_T / 64), sc.run, sc.noted, sc.st);
+    } else {
+        k_chain_sum<<<1, SQ_T, SQ_LDS, st>>>(sc.e, n, sc.st);
+    }
+    uint32_t *key = (uint32_t *)sc.kin, *sorted = (uint32_t *)sc.kout;
+    int *id = (int *)sc.kin + n, *pi = (int *)sc.kout + n;
+    k_sample_keys<<<nb, NT, 0, st>>>(sc.e, n, cutoff, sc.st, key, id);
     if (mhip::check_launch(c, "sampler")) return -1;
     size_t tb = sc.tmp_bytes;
-    if (mhip::check(c, rocprim::radix_sort_keys(sc.tmp, tb, sc.kin, sc.kout, (unsigned)n, 0, 64, st),
+    if (mhip::check(c, rocprim::radix_sort_pairs(sc.tmp, tb, key, sorted, id, pi, (unsigned)n, 0, 32, st),
                     "sampler sort"))
         return -1;
     float *pf = (float *)sc.kin;  // the unsorted keys are dead after the sort
-    int *pi = (int *)sc.kin + n;
-    k_keys_split<<<nb, NT, 0, st>>>(sc.kout, n, pf, pi, sc.st);
+    k_keys_split<<<nb, NT, 0, st>>>(sorted, n, pf, sc.st);
     k_sample_pick<<<1, SQ_T, SQ_LDS, st>>>(pf, pi, s->top_p, u, sc.st, d_token);
     return mhip::check_launch(c, "sampler pick");
 }

@@ -155,6 +155,36 @@ def test_model_generation_step_sample(oracle, tmp_path, t, p):
         b.close()
 
 
+@pytest.mark.parametrize("n", [2047, 2048, 2049, 4097, 151936, 524288, 524289])
+def test_sampler_sum_over_the_chip(oracle, gpu, n):
+    """From 2048 to 524288 logits the sum of the exponentials is composed of
+    256-thread workgroups' runs, outside those sizes taken on one workgroup:
+    spread logits, equal ones (every sum exact, powers of two met exactly),
+    two values (ties), a ramp over the whole range of exp (zeros, subnormals,
+    many binades), a late maximum, -inf and NaN."""
+    say("test_sampler_sum_over_the_chip n=%d" % n)
+    rng = np.random.default_rng(n)
+    spread = (rng.standard_normal(n) * 3).astype(np.float32)
+    late = spread.copy()
+    late[-1] = 40.0
+    some = spread.copy()
+    some[rng.integers(0, n, n // 3)] = -np.inf
+    nan = spread.copy()
+    nan[n // 2] = np.nan
+    ds = DevSampler(gpu, n)
+    try:
+        for name, lg in (("spread", spread), ("equal", np.zeros(n, np.float32)),
+                         ("two", np.where(rng.random(n) < 0.5, 0.0, -0.6931472).astype(np.float32)),
+                         ("ramp", np.linspace(-110, 0, n).astype(np.float32)),
+                         ("fall", np.linspace(0, -110, n).astype(np.float32)),
+                         ("late", late), ("-inf", some), ("nan", nan)):
+            for t, p in ((1.0, 1.0), (0.7, 0.9)):
+                got, _ = ds.draws(lg, t, p, 11, 3)
+                assert got == oracle.sample(lg, t, p, 11, 3), (name, t, p)
+    finally:
+        ds.close()
+
+
 def _chain_cases():
     """Vectors for the running sums: (name, values, thresholds)."""
     rng = np.random.default_rng(31)
