@@ -52,7 +52,7 @@ int mia_gpu_model_feed(mia_gpu_model *m, int token, int pos);
 
 /* n feeds in one call (no counterpart in the reference, whose serve loop
  * feeds a prompt one token at a time): tokens[0..n) at positions
- * pos .. pos + n - 1, in batches of equal size (at most 1024 tokens)
+ * pos .. pos + n - 1, in batches of equal size (at most 2048 tokens)
  * through each layer at once (the attention of the batch with
  * mhip_attention_batch, its MoE on the per-stage kernels for T tokens, the
  * matrix-core ones from MHIP_GEMM_MIN_A assignments on), so the weights are

@@ -414,7 +414,8 @@ void launch_attn_batch(hipStream_t st, const float *q, const float *kc, const fl
     const int group = nh / nkv, kvd = nkv * HD, qd = nh * HD;
     const int sld = (pos + n + 3) & ~3, pld = part_ld(sld);
     const size_t fit = (bytes - 3 * 256) / token_bytes(nh, sld);
-    const int pass = fit < (size_t)n ? (int)fit : n;
+    // passes of equal size
+    const int np = fit < (size_t)n ? (int)((n + fit - 1) / fit) : 1, pass = (n + np - 1) / np;
     float *S = (float *)scratch;
     float *pmax = (float *)((uint8_t *)S + align256((size_t)pass * nh * sld * 4));
     float2 *stat = (float2 *)((uint8_t *)pmax + align256((size_t)pass * nh * pld * 4));
