@@ -914,6 +914,10 @@ int mhip_attention_batch(mhip_ctx *c, const mhip_attn_dims *s, const float *d_at
     if (n <= 0 || pos < 0 || pos + n > max_seq)
         return mhip::fail(c, "attention batch: positions %d .. %d outside [0, max_seq=%d)", pos,
                           pos + n - 1, max_seq);
+    for (const void *p : {(const void *)d_attn_norm, d_wq, d_wk, d_wv, d_wo, (const void *)d_q_norm,
+                          (const void *)d_k_norm, (const void *)d_rope, (const void *)d_kc,
+                          (const void *)d_vc, (const void *)d_x, (const void *)d_scratch})
+        if (!p) return mhip::fail(c, "attention batch: a null argument");
     if (mhip::use_device(c)) return -1;
     const int d = s->dim, nh = s->n_heads, nkv = s->n_kv_heads, hd = s->head_dim;
     const int qd = nh * hd, kvd = nkv * hd, nb = d / QK;

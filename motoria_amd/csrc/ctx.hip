@@ -181,7 +181,10 @@ const char *mhip_error(const mhip_ctx *c) { return c ? c->err : "null context"; 
 void *mhip_malloc(mhip_ctx *c, size_t bytes) {
     if (mhip::use_device(c)) return nullptr;
     void *p = nullptr;
-    if (mhip::check(c, hipMalloc(&p, bytes ? bytes : 1), "hipMalloc")) return nullptr;
+    if (mhip::check(c, hipMalloc(&p, bytes ? bytes : 1), "hipMalloc")) {
+        (void)hipGetLastError();  // reported here: not by the next launch's check
+        return nullptr;
+    }
     return p;
 }
 
@@ -213,8 +216,10 @@ void *mhip_host_malloc(mhip_ctx *c, size_t bytes) {
     if (mhip::use_device(c)) return nullptr;
     void *p = nullptr;
     if (mhip::check(c, hipHostMalloc(&p, bytes ? bytes : 1, hipHostMallocDefault),
-                    "hipHostMalloc"))
+                    "hipHostMalloc")) {
+        (void)hipGetLastError();
         return nullptr;
+    }
     return p;
 }
 

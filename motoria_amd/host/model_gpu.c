@@ -538,11 +538,18 @@ int mia_gpu_model_prefill(mia_gpu_model *m, const int *tokens, int n, int pos) {
     const size_t kvd = (size_t)h->n_kv_heads * h->head_dim, row = (size_t)(d / MIA_QK) * 36;
     const int bmax = prefill_max(h);
     if (n == 0) return 0;
-    if (!m->d_xb) {
+    if (!m->d_bscratch) {
+        /* both or neither, so that a call after a failed one starts over */
         m->d_xb = mhip_malloc(m->gpu, (size_t)bmax * d * 4);
-        m->d_bscratch =
-            mhip_malloc(m->gpu, mhip_attention_batch_scratch_bytes(&m->ad, bmax, m->max_seq));
-        if (!m->d_xb || !m->d_bscratch) return mfail(m, "device memory: %s", mhip_error(m->gpu));
+        if (m->d_xb)
+            m->d_bscratch =
+                mhip_malloc(m->gpu, mhip_attention_batch_scratch_bytes(&m->ad, bmax, m->max_seq));
+        if (!m->d_bscratch) {
+            mfail(m, "device memory: %s", mhip_error(m->gpu));
+            mhip_free(m->gpu, m->d_xb);
+            m->d_xb = NULL;
+            return -1;
+        }
         /* the attention weights packed once for the matrix-core rows; a
          * shape they do not fit keeps the vector rows */
         const size_t pb = mhip_attention_pack_bytes(&m->ad);

@@ -175,3 +175,27 @@ def test_batch_with_infinities():
         assert torch.equal(torch.isfinite(got), torch.isfinite(want))
     finally:
         lay.close()
+
+
+def test_batch_refuses_null():
+    """A missing buffer (the scratch of a failed allocation, say) is an error
+    of the call, not a launch."""
+    torch = pytest.importorskip("torch")
+    say("test_batch_refuses_null")
+    lay = Layer(torch, 256, 8, 2, 16, 3)
+    try:
+        kc, vc = lay.cache(4)
+        x = lay.up(np.ones((2, 256), np.float32))
+        nb = lay.L.mhip_attention_batch_scratch_bytes(ctypes.byref(lay.a), 2, 16)
+        scratch = torch.zeros(nb, dtype=torch.uint8, device="cuda")
+        torch.cuda.synchronize()
+        ptrs = lay.args(kc, vc)
+        for miss in range(len(ptrs) + 2):
+            p = [None if i == miss else v for i, v in enumerate(ptrs)]
+            rc = lay.L.mhip_attention_batch(
+                lay.g.h, ctypes.byref(lay.a), *p, 4, 2, 16,
+                None if miss == len(ptrs) else x.data_ptr(), lay.pack.data_ptr(),
+                None if miss == len(ptrs) + 1 else scratch.data_ptr(), 0)
+            assert rc == -1 and b"null" in lay.L.mhip_error(lay.g.h), miss
+    finally:
+        lay.close()
