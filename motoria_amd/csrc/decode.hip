@@ -1722,7 +1722,7 @@ int mhip_decode_in(mhip_ctx *c, float *d_x, const float *h_x, int d) {
 
 int mhip_decode_out(mhip_ctx *c, const void *d_ws, const float *d_x, int d, const int *d_idx,
                     const float *d_w, int nr, void *h_out, int status[4]) {
-    if (d <= 0 || nr < 0 || !d_ws || !d_x || !h_out)
+    if (d <= 0 || nr < 0 || !d_ws || !d_x || !h_out || !status || (nr > 0 && (!d_idx || !d_w)))
         return mhip::fail(c, "decode out: bad arguments (d=%d, nr=%d)", d, nr);
     if (mhip::use_device(c)) return -1;
     const int m = d > nr ? d : nr;

@@ -281,3 +281,35 @@ def test_decode_rejects_more_than_256_layers(qwen_dims, moe):
                              None, None, None, None, M.DECODE_MAX_LAYERS + 1, None, None, None, 0)
     assert rc == -1
     assert b"outside [0, 256]" in L.mhip_error(moe.gpu)
+
+
+def test_decode_out_refuses_null():
+    """mhip_decode_in / mhip_decode_out: a missing buffer is an error of the
+    call, not a launch; with no routing asked for, its buffers may be null."""
+    say("test_decode_out_refuses_null")
+    g, L, d, nr = M.Gpu(), M.lib(), 64, 8
+    try:
+        ws, x = g.malloc(L.mhip_decode_ws_bytes()), g.upload(np.arange(d, dtype=np.float32))
+        idx, w = g.upload(np.arange(nr, dtype=np.int32)), g.upload(np.ones(nr, np.float32))
+        h = L.mhip_host_malloc(g.h, (d + 2 * nr + 6) * 4)
+        st = (ctypes.c_int * 4)()
+        g.check(L.mhip_zero(g.h, ws, L.mhip_decode_ws_bytes()), "zero")
+
+        def out(ws, x, idx, w, nr, h, st):
+            return L.mhip_decode_out(g.h, ws, x, d, idx, w, nr, h, st)
+
+        good = [ws, x, idx, w, nr, h, st]
+        for miss in (0, 1, 2, 3, 5, 6):
+            assert out(*[None if i == miss else v for i, v in enumerate(good)]) == -1, miss
+        assert L.mhip_decode_in(g.h, None, h, d) == -1 and L.mhip_decode_in(g.h, x, None, d) == -1
+        g.check(out(*good), "decode out")
+        words = np.ctypeslib.as_array(ctypes.cast(h, ctypes.POINTER(ctypes.c_uint32)), (d + 2 * nr,))
+        assert np.array_equal(words[:d].view(np.float32), np.arange(d))
+        assert np.array_equal(words[d:d + nr], np.arange(nr))
+        assert list(st) == [0, 0, 0, 0]
+        g.check(out(ws, x, None, None, 0, h, st), "decode out without routing")
+        L.mhip_host_free(g.h, h)
+        for p in (ws, x, idx, w):
+            g.free(p)
+    finally:
+        g.close()
