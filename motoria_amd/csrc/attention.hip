@@ -595,9 +595,9 @@ __global__ __launch_bounds__(256) void k_attn_mix_b(float *__restrict__ scores, 
 // 0 .. group - 1 of wavefront 0, one head each. Mix: thread (element
 // tid % AG_HD, heads tid / AG_HD + 2 j), the value rows read 16 positions
 // ahead of their additions. Scores (row stride sld, a multiple of 4) in
-// LDS behind the key rows: below AB_MIN_CTX positions they always fit.
+// LDS behind the key rows (tiles_fit: the calls that come here fit).
 constexpr int AG_HD = 128, AG_KLD = AG_HD + 4, AG_MAXG = 16;
-constexpr size_t AG_LDS_MAX = 150 * 1024;
+constexpr size_t AG_LDS_MAX = 150 * 1024, AG_LDS_STATIC = 32 * 8 + AG_MAXG * 4;
 size_t ag_lds(int group, int sld) {
     return (size_t)(256 / group) * AG_KLD * 4 + (size_t)group * sld * 4;
 }
@@ -734,12 +734,27 @@ __global__ __launch_bounds__(256) void k_attn_group_b(const float *__restrict__ 
 // us, workgroup per token / tiles): 8 tokens at 600 162/164, at 1000 209/208,
 // at 2000 353/315; 100 at 600 207/208, at 1000 259/255, at 2000 601/381; at
 // position 0 200 tokens 209/209, 300 277/270, 500 435/406.
-constexpr int AB_MIN_CTX = 1000, AB_MIN_N = 250;
+// Few heads leave the tiles without enough rows for the chip: with one head to
+// a group, or up to 8 heads in groups of up to 4, the workgroup per token stays
+// while all of them are resident at once. In a 16-layer model (so with the
+// caches not in L2), us a layer, at 1500: 16/16 heads 16 tokens 267/283, 32 (two
+// rounds of workgroups) 367/305; 4/4 heads 64 tokens 275/328, 96 392/365; 8/2
+// heads 16 tokens 246/269; but 16/8 heads 16 tokens 292/279, 16/4 280/276, 32/8
+// 329/293.
+constexpr int AB_MIN_CTX = 1000, AB_MIN_N = 250, AB_FEW = 8, AB_FEW_G = 4;
+constexpr size_t NCU = 256, CU_LDS = 160 * 1024;
 static_assert((256 * AG_KLD + AB_MIN_CTX) * 4 <= AG_LDS_MAX &&
                   (256 / AG_MAXG * AG_KLD + AG_MAXG * AB_MIN_CTX) * 4 <= AG_LDS_MAX,
               "k_attn_group_b's scores fit LDS at every group");
 bool tiles_fit(const mhip_attn_dims *s, int n, int end) {
-    return s->head_dim == AG_HD && (end >= AB_MIN_CTX || n >= AB_MIN_N);
+    if (s->head_dim != AG_HD) return false;
+    const int group = s->n_heads / s->n_kv_heads;
+    const size_t lds = ag_lds(group, (end + 3) & ~3);
+    if ((group == 1 || (s->n_heads <= AB_FEW && group <= AB_FEW_G)) && 256 % group == 0 &&
+        lds <= AG_LDS_MAX &&
+        (size_t)n * s->n_kv_heads <= NCU * (CU_LDS / (lds + AG_LDS_STATIC)))
+        return false;
+    return end >= AB_MIN_CTX || n >= AB_MIN_N;
 }
 
 constexpr size_t HEAD_LDS_MAX = 150 * 1024;  // dynamic LDS of k_attn_head
@@ -863,7 +878,9 @@ static size_t scores_bytes(const mhip_attn_dims *s, int n, int max_seq) {
 }
 
 size_t mhip_attention_batch_scratch_bytes(const mhip_attn_dims *s, int n, int max_seq) {
-    if (!s || n <= 0 || max_seq <= 0) return 0;
+    if (!s || n <= 0 || max_seq <= 0 || s->n_heads <= 0 || s->n_kv_heads <= 0 ||
+        s->n_heads % s->n_kv_heads)
+        return 0;
     const size_t d = s->dim, qd = (size_t)s->n_heads * s->head_dim,
                  kvd = (size_t)s->n_kv_heads * s->head_dim, N = (size_t)n,
                  P = (N + 127) & ~(size_t)127;

@@ -2,11 +2,12 @@
 attention (mhip_attention, src/model/forward.c:118-165 of the reference) at
 every token: outputs and cache rows bit for bit.
 
-From 250 tokens or 1000 positions on (head_dim 128) the scores and the mix
-run in tiles of 64 x 64 and 32 x 32 (rows x positions; a row is a token and
-a head of its key/value group), the softmax sums 128 positions at a time,
-and batches of long contexts in passes of a bounded score matrix: the sizes
-lie around those edges, over groups of 8, 1, 3 and 10 heads. Cache rows past the batch
+From 250 tokens or 1000 positions on (head_dim 128; few heads later) the
+scores and the mix run in tiles of 64 x 64 and 32 x 32 (rows x positions; a
+row is a token and a head of its key/value group), the softmax sums 128
+positions at a time, and batches of long contexts in passes of a bounded
+score matrix: the sizes lie around those edges, over groups of 8, 1, 3 and
+10 heads. Cache rows past the batch
 and the scratch are NaN before the call."""
 import ctypes
 
@@ -112,6 +113,29 @@ def test_batch_equals_tokens(n, pos, nh, nkv):
         assert np.array_equal(bits(got), bits(want)), "matrix-core rows"
         assert np.array_equal(bits(kc[:pos + n]), bits(k2[:pos + n]))
         assert np.array_equal(bits(vc[:pos + n]), bits(v2[:pos + n]))
+    finally:
+        lay.close()
+
+
+@pytest.mark.parametrize("nh,nkv,n,pos", [
+    (4, 4, 64, 1000), (4, 4, 65, 1000), (8, 4, 128, 1000), (8, 4, 129, 1000), (8, 2, 384, 700),
+    (8, 2, 385, 700), (1, 1, 1, 4607), (1, 1, 1, 4608), (4, 1, 2, 7486), (4, 1, 2, 7487)])
+def test_batch_of_few_heads(n, pos, nh, nkv):
+    """Few heads, in groups of one, two and four: a workgroup per token while
+    all of them are resident at once, tiles from one token more; the longest
+    contexts whose scores fit LDS, and the next."""
+    torch = pytest.importorskip("torch")
+    say("test_batch_of_few_heads n=%d pos=%d heads %d/%d" % (n, pos, nh, nkv))
+    lay = Layer(torch, 256, nh, nkv, pos + n, n + pos)
+    try:
+        kc, vc = lay.cache(pos)
+        k2, v2 = kc.clone(), vc.clone()
+        x = lay.up(lay.rng.standard_normal((n, 256)).astype(np.float32))
+        want = torch.cat([lay.token(x[i:i + 1], k2, v2, pos + i) for i in range(n)])
+        assert torch.isfinite(want).all()
+        for packed in (False, True):
+            got = lay.batch(x, kc.clone(), vc.clone(), pos, packed=packed)
+            assert np.array_equal(bits(got), bits(want)), packed
     finally:
         lay.close()
 
