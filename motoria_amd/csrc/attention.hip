@@ -501,7 +501,9 @@ __global__ __launch_bounds__(256) void k_qk_rope_b128(float *__restrict__ q,
     if (h >= nh + 2 * nkv) return;
     if (h >= nh + nkv) {
         const size_t o = (size_t)(h - nh - nkv) * QR_HD + 2 * lane;
-        *(float2 *)(vc + (size_t)p * kvd + o) = *(const float2 *)(v + (size_t)t * kvd + o);
+        const float2 r = *(const float2 *)(v + (size_t)t * kvd + o);
+        vc[(size_t)p * kvd + o] = r.x;
+        vc[(size_t)p * kvd + o + 1] = r.y;
         return;
     }
     const bool isq = h < nh;
@@ -511,7 +513,8 @@ __global__ __launch_bounds__(256) void k_qk_rope_b128(float *__restrict__ q,
                      : kc + (size_t)p * kvd + (size_t)(h - nh) * QR_HD;
     const float *w = isq ? q_norm : k_norm;
     const float r0 = src[lane], r1 = src[lane + 64], w0 = w[lane], w1 = w[lane + 64];
-    const double2 cs = *(const double2 *)(rope + ((size_t)p * (QR_HD / 2) + lane) * 2);
+    const double *rp = rope + ((size_t)p * (QR_HD / 2) + lane) * 2;  // (8-byte aligned, no more)
+    const double cs = rp[0], sn = rp[1];
     double ss = (double)r0 * (double)r0 + (double)r1 * (double)r1;
     ss = mhip_attn::readlane_d(mhip_attn::wave_sum63(ss), 63);
     const double m = ss * ((double)(QR_HD + 64) * 0x1p-52);
@@ -526,8 +529,8 @@ __global__ __launch_bounds__(256) void k_qk_rope_b128(float *__restrict__ q,
         inv = (float)(1.0 / sqrt(sq / QR_HD + (double)eps));
     }
     const float x0 = (r0 * inv) * w0, x1 = (r1 * inv) * w1;
-    dst[lane] = (float)((double)x0 * cs.x - (double)x1 * cs.y);
-    dst[lane + 64] = (float)((double)x0 * cs.y + (double)x1 * cs.x);
+    dst[lane] = (float)((double)x0 * cs - (double)x1 * sn);
+    dst[lane + 64] = (float)((double)x0 * sn + (double)x1 * cs);
 }
 
 // k_attn_scores for token blockIdx.y: scores[t][h][0 .. pos + t].

@@ -30,6 +30,7 @@ namespace {
 
 constexpr int HD = 128;
 typedef float f4v __attribute__((ext_vector_type(4)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));  // of a caller's cache rows
 typedef float f16v __attribute__((ext_vector_type(16)));
 
 // acc += p; gives `next` back for a product that then does not start before
@@ -125,7 +126,7 @@ __global__ __launch_bounds__(256, 4) void k_ab_scores(const float *__restrict__ 
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         qv[k] = *(const f4v *)(qb + qp[k]);
-        kv[k] = *(const f4v *)(kb + kp[k]);
+        kv[k] = *(const f4u *)(kb + kp[k]);
     }
     f16v acc = {0.0f};
     const f4v *A = (const f4v *)&qs[(wr + 16 * (blk >> 1) + c16) * SLD];
@@ -143,7 +144,7 @@ __global__ __launch_bounds__(256, 4) void k_ab_scores(const float *__restrict__ 
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 qv[k] = *(const f4v *)(qb + i0 + SI + qp[k]);
-                kv[k] = *(const f4v *)(kb + i0 + SI + kp[k]);
+                kv[k] = *(const f4u *)(kb + i0 + SI + kp[k]);
             }
         }
         // the products of a term are formed while the previous term's are added
@@ -307,7 +308,7 @@ __global__ __launch_bounds__(256, 4) void k_ab_mix(const float *__restrict__ S, 
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             const int w = min(u0 + (tid >> 5) + 8 * k, np - 1);  // (past the end: not used)
-            vv[k] = *(const f4v *)(vp + (size_t)w * kvd);
+            vv[k] = *(const f4u *)(vp + (size_t)w * kvd);
         }
     };
     fetch(0);

@@ -27,6 +27,7 @@ namespace {
 constexpr int QK = mhip::QK;
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float f4v __attribute__((ext_vector_type(4)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));  // of a caller's x
 
 constexpr int RM_R = 64;  // weight rows of a workgroup
 constexpr int FRAG = 16 * QK;  // codes of a fragment
@@ -181,8 +182,8 @@ __global__ __launch_bounds__(256, 4) void k_rows_mfma(RowPack sg, int nb, int n,
             for (int i = 0; i < 2; i++) {
                 const int row = rl0 + 16 * (wr + i) + 4 * c;
                 f4v v = acc[i][j];
-                if (resid) v = *(const f4v *)(resid + (size_t)t * ld_r + row) + v;
-                *(f4v *)(sg.out[k] + (size_t)t * R + row) = v;
+                if (resid) v = *(const f4u *)(resid + (size_t)t * ld_r + row) + v;
+                *(f4u *)(sg.out[k] + (size_t)t * R + row) = v;
             }
         }
     }

@@ -201,6 +201,41 @@ def test_batch_with_infinities():
         lay.close()
 
 
+@pytest.mark.parametrize("n,pos", [(5, 30), (40, 1000)])
+def test_batch_on_unaligned_buffers(n, pos):
+    """x and the value rows at a multiple of 4 bytes, the rotation angles at
+    one of 8: what float and double pointers promise."""
+    torch = pytest.importorskip("torch")
+    say("test_batch_on_unaligned_buffers n=%d pos=%d" % (n, pos))
+    lay = Layer(torch, 256, 8, 2, pos + n, n)
+    try:
+        kc, vc = lay.cache(pos)
+        x = lay.up(lay.rng.standard_normal((n, 256)).astype(np.float32))
+        k2, v2 = kc.clone(), vc.clone()
+        want = lay.batch(x, k2, v2, pos)
+
+        def shifted(t):
+            b = torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")
+            b[1:] = t.reshape(-1)
+            return b
+
+        xs, vs, rope = shifted(x), shifted(vc), shifted(lay.rope)
+        nb = lay.L.mhip_attention_batch_scratch_bytes(ctypes.byref(lay.a), n, pos + n)
+        scratch = torch.zeros(nb, dtype=torch.uint8, device="cuda")
+        torch.cuda.synchronize()
+        args = lay.args(kc, vc)
+        args[7], args[9] = rope[1:].data_ptr(), vs[1:].data_ptr()
+        lay.g.check(lay.L.mhip_attention_batch(
+            lay.g.h, ctypes.byref(lay.a), *args, pos, n, pos + n, xs[1:].data_ptr(),
+            lay.pack.data_ptr(), scratch.data_ptr(), 0), "batch")
+        torch.cuda.synchronize()
+        assert np.array_equal(bits(xs[1:].reshape(n, 256)), bits(want))
+        assert np.array_equal(bits(kc), bits(k2))
+        assert np.array_equal(bits(vs[1:].reshape(vc.shape)), bits(v2))
+    finally:
+        lay.close()
+
+
 def test_batch_refuses_null():
     """A missing buffer (the scratch of a failed allocation, say) is an error
     of the call, not a launch."""
