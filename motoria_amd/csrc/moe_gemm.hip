@@ -76,7 +76,7 @@ struct alignas(16) Step {
     _Float16 x[TM][KB];  // 8 KB
     int8_t w[TN][KB];    // 8 KB
     float sw[TN];        // 1 KB
-    float sx[TM];        // 512 B: the scale of bucket row 16 j + l at 8 l + j
+    float sx[TM];        // 512 B: the scale of row 16 j + l at 8 l + j
 };
 static_assert(sizeof(Step) == 17920, "step layout");
 
@@ -265,30 +265,41 @@ __device__ __forceinline__ void step(const char *S, const Lanes &la, int nstep,
 }
 
 // A wavefront's place in a tile. A heavy tile (over TM / 2 rows): weight rows
-// 64 (w % 4) .. + 63, the assignment rows' half w / 4. A light one: 32 weight
-// rows against all its rows.
+// 64 (w % 4) .. + 63, half w / 4 of the assignment tiles (of an odd count the
+// second half's last one is empty, so that every wavefront of the workgroup
+// runs the same code and meets the same barriers). A light one: 32 weight rows
+// against all its rows.
 struct Place {
     bool heavy;
-    int n0, j0, nj;  // LDS weight row of its first tile; assignment tiles j0 .. + nj
+    int n0, j0;      // LDS weight row, LDS assignment tile of its first tiles
+    int r0, nj;      // its assignment tiles r0 .. + nj of the bucket's
 };
+// The assignment tiles of the halves of a heavy tile, and the bucket row at
+// row m of the ring: the second half starts at ring tile NJ.
+__device__ __forceinline__ int half_tiles(int nrows) { return (nrows + 31) / 32; }
+__device__ __forceinline__ int ring_row(int m, int nrows) {
+    const int r = nrows > TM / 2 && m >= TM / 2 ? m - TM / 2 + 16 * half_tiles(nrows) : m;
+    return min(r, nrows - 1);  // (past the end: a valid row, its results unused)
+}
 __device__ __forceinline__ Place place_of(int nrows, int wave, bool paired) {
     Place p;
     p.heavy = nrows > TM / 2;
     if (p.heavy) {
         p.n0 = WN * (wave & 3);
+        p.nj = half_tiles(nrows);
         p.j0 = NJ * (wave >> 2);
-        p.nj = min(NJ, (nrows + 15) / 16 - p.j0);
+        p.r0 = p.nj * (wave >> 2);
     } else {
         // gate/up pairs a gate tile with the up tile 32 rows on
         p.n0 = paired ? WN * (wave >> 1) + 16 * (wave & 1) : 32 * wave;
-        p.j0 = 0;
+        p.j0 = p.r0 = 0;
         p.nj = (nrows + 15) / 16;
     }
     return p;
 }
 
 // The k loop over nk steps (nk >= NS - 1). On return acc[NJ i + j][r] holds
-//   C[n0 + 16 i + 4 (lane / 16) + r][16 (j0 + j) + lane % 16]
+//   C[n0 + 16 i + 4 (lane / 16) + r][16 (r0 + j) + lane % 16]
 // (weight row, assignment row; a light tile's second weight tile lies NSTEP
 // rows on) for j < nj: the exact block dots, each block
 // term added with its two scales in block order.
@@ -336,19 +347,16 @@ __device__ __forceinline__ void gemm_tile(Step *ring, const Src &src, int nk, co
     __syncthreads();
 }
 
-// The k loop in the form of the wavefront's place: one per count of 16-row
-// assignment tiles, so a bucket's last tile runs no empty tile. (The two
-// halves of a heavy tile may take different forms: the choice is a
-// wavefront's, and every form meets nk + 1 barriers.)
+// The k loop in the form of the tile (every wavefront of the workgroup the
+// same): one per count of 16-row assignment tiles of a wavefront, so a
+// bucket's last tile runs at most one empty tile.
 template <bool EXACT, int NSTEP>
 __device__ __forceinline__ void gemm_tile_rows(Step *ring, const Src &src, int nk, const Place &pl,
                                                f4v (&acc)[MI * NJ]) {
     if (pl.heavy) {
         switch (pl.nj) {
         case 4: gemm_tile<EXACT, MI, 4, 16>(ring, src, nk, pl, acc); break;
-        case 3: gemm_tile<EXACT, MI, 3, 16>(ring, src, nk, pl, acc); break;
-        case 2: gemm_tile<EXACT, MI, 2, 16>(ring, src, nk, pl, acc); break;
-        default: gemm_tile<EXACT, MI, 1, 16>(ring, src, nk, pl, acc); break;
+        default: gemm_tile<EXACT, MI, 3, 16>(ring, src, nk, pl, acc); break;
         }
     } else {
         switch (pl.nj) {
@@ -428,7 +436,7 @@ __global__ __launch_bounds__(GT, 4) void k_gateup_mfma(
     Src src;
     {
         const Pieces p = pieces();
-        src.x = xq16 + (size_t)(perm[base + min(p.xr, nrows - 1)] / K) * d + p.xc * 8;
+        src.x = xq16 + (size_t)(perm[base + ring_row(p.xr, nrows)] / K) * d + p.xc * 8;
         // tile row n: wavefront n / 64; within it gate rows then up rows
         auto wrow = [&](int n, int half) {
             const int r = n % WN;
@@ -443,8 +451,8 @@ __global__ __launch_bounds__(GT, 4) void k_gateup_mfma(
             src.s = (const float *)(ex + (lane < WN / 2 ? lay.gate_st : lay.up_st)) + hc;
             src.sstep = eh;
         } else {
-            // sx slot p holds bucket row 16 (p % 8) + p / 8
-            src.s = xsb + base + min(16 * (p.sx & 7) + (p.sx >> 3), nrows - 1);
+            // sx slot p holds ring row 16 (p % 8) + p / 8
+            src.s = xsb + base + ring_row(16 * (p.sx & 7) + (p.sx >> 3), nrows);
             src.sstep = A;
         }
     }
@@ -467,7 +475,7 @@ __global__ __launch_bounds__(GT, 4) void k_gateup_mfma(
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
         if (j < pl.nj) {
-            const int row = 16 * (pl.j0 + j) + l16;
+            const int row = 16 * (pl.r0 + j) + l16;
             if (pl.heavy) {
 #pragma unroll
                 for (int i = 0; i < MI / 2; i++)
@@ -541,14 +549,14 @@ __global__ __launch_bounds__(GT, 4) void k_down_mfma(const uint8_t *__restrict__
     Src src;
     {
         const Pieces p = pieces();
-        src.x = hq16 + (size_t)(base + min(p.xr, nrows - 1)) * eh + p.xc * 8;
+        src.x = hq16 + (size_t)(base + ring_row(p.xr, nrows)) * eh + p.xc * 8;
         src.w = (const int8_t *)(ex + lay.down_q) + (size_t)(n0 + p.wr) * eh + 16 * p.wh;
         if (wave < 4) {
             src.s = (const float *)(ex + lay.down_st) + n0 + WN * wave + lane;
             src.sstep = d;
         } else {
-            // sx slot p holds bucket row 16 (p % 8) + p / 8
-            src.s = hsb + base + min(16 * (p.sx & 7) + (p.sx >> 3), nrows - 1);
+            // sx slot p holds ring row 16 (p % 8) + p / 8
+            src.s = hsb + base + ring_row(16 * (p.sx & 7) + (p.sx >> 3), nrows);
             src.sstep = A;
         }
     }
@@ -570,7 +578,7 @@ __global__ __launch_bounds__(GT, 4) void k_down_mfma(const uint8_t *__restrict__
 #pragma unroll
                     for (int i = 0; i < MI; i++)
                         if (pl.heavy || i < MI / 2)
-                            *(f4v *)&L.o[16 * (pl.j0 + j) + l16][pl.n0 % (TN / 2) + 16 * i + 4 * c] =
+                            *(f4v *)&L.o[16 * (pl.r0 + j) + l16][pl.n0 % (TN / 2) + 16 * i + 4 * c] =
                                 acc[i * NJ + j];
                 }
         }

@@ -295,6 +295,29 @@ def test_layer_skewed_2048(oracle, qwen_dims, qwen_moe):
     assert 0.35 < share4 < 0.5 and 20 <= zero <= 40
 
 
+@pytest.mark.parametrize("T", [600, 1301, 2048])
+def test_layer_every_tile_form(oracle, qwen_dims, qwen_moe, T):
+    """The matrix-core expert products against the vector kernels (bits), on
+    buckets whose last tiles hold every count of 16-row groups, 1 to 8, and
+    rows that are not whole groups."""
+    say("test_layer_every_tile_form T=%d" % T)
+    x = oracle.synth_x(W.X_SEED + T, T, qwen_dims.dim)
+    bias = (0.6 * W.zipf_bias(qwen_dims.n_experts)).astype(np.float32)
+    n0 = M.lib().mhip_matrix_layers(qwen_moe.gpu)
+    xm, im, wm, _ = _gpu_layer(qwen_moe, 0, x, bias, 0)
+    assert M.lib().mhip_matrix_layers(qwen_moe.gpu) == n0 + 1
+    xv, iv, wv, _ = _gpu_layer(qwen_moe, 0, x, bias, M.MHIP_EXACT_EXPERTS)
+    assert M.lib().mhip_matrix_layers(qwen_moe.gpu) == n0 + 1
+    cnt = np.bincount(im.ravel(), minlength=qwen_dims.n_experts)
+    last = (cnt[cnt > 0] - 1) % 128 + 1
+    forms = set(((last + 15) // 16).tolist())
+    assert forms == set(range(1, 9)), forms
+    assert np.any(last % 16)
+    assert np.array_equal(im, iv)
+    assert_bits(wm, wv, "gate weights")
+    assert_bits(xm, xv, "layer output")
+
+
 def _every_token(oracle, d, T, seed, bias=None):
     """One matrix-core layer at T tokens on a fresh one-layer handle with a
     non-unit ffn_norm: every token's logits, expert indices, gate weights and
