@@ -30,7 +30,7 @@ constexpr uint32_t NONE = ~0u;    // key of a dropped token
 struct SampleState {
     int best;
     float sum;
-    int token;
+    int walked;  // how the sum was taken: pieces that k_sum_walk noted, -1 by seq_scan alone
     int last;
     float cum;
 };
@@ -375,7 +375,10 @@ __global__ __launch_bounds__(SQ_T) void k_chain_sum(const float *__restrict__ e,
                                                     SampleState *st) {
     float s;
     seq_scan<SQ_SUM>(e, n, 0.0f, &s);
-    if (threadIdx.x == 0) st->sum = s;
+    if (threadIdx.x == 0) {
+        st->sum = s;
+        st->walked = -1;
+    }
 }
 
 // ---- the same over the whole chip ---------------------------------------------------
@@ -559,6 +562,7 @@ __global__ __launch_bounds__(SQ_T) void k_sum_walk(const float *__restrict__ e, 
             }
             if (tid == 0) {
                 st->sum = s;
+                st->walked = total;
                 bad = !ok;
             }
         }
@@ -567,7 +571,10 @@ __global__ __launch_bounds__(SQ_T) void k_sum_walk(const float *__restrict__ e, 
     }
     float s;
     seq_scan<SQ_SUM>(e, n, 0.0f, &s);
-    if (tid == 0) st->sum = s;
+    if (tid == 0) {
+        st->sum = s;
+        st->walked = -1;
+    }
 }
 
 // sampler.c:46-51: p_i = e_i / sum; a candidate when p_i >= cutoff, as the

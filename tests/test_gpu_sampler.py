@@ -185,6 +185,78 @@ def test_sampler_sum_over_the_chip(oracle, gpu, n):
         ds.close()
 
 
+def _sum_cases(n):
+    """(name, logits, temperature): model-like logits over many seeds (the
+    spread values are ties in a share of their additions), equal ones (a sum of
+    ones meets every power of two exactly), two and three values in blocks and
+    at random (sums just below and above the powers), a ramp up and down the
+    whole range of exp (zeros, subnormals, more pieces than the walk takes),
+    a late maximum, -inf and NaN."""
+    rng = np.random.default_rng(n)
+    out = []
+    for seed in range(24):
+        lg = (rng.standard_normal(n) * 2.5).astype(np.float32)
+        lg[rng.integers(0, n, 40)] += (8.0 + 6.0 * rng.random(40)).astype(np.float32)
+        out.append(("model %d" % seed, lg, (0.6, 0.8, 1.0)[seed % 3]))
+    spread = (rng.standard_normal(n) * 3).astype(np.float32)
+    out.append(("spread", spread, 1.0))
+    out.append(("equal", np.zeros(n, np.float32), 1.0))
+    half, third = np.float32(-0.6931472), np.float32(-1.0986123)
+    out.append(("two", np.where(rng.random(n) < 0.5, np.float32(0), half).astype(np.float32), 1.0))
+    blocks = np.where(np.arange(n) // 37 % 2 == 0, np.float32(0), half)
+    out.append(("blocks", blocks.astype(np.float32), 1.0))
+    out.append(("three", rng.choice([np.float32(0), half, third], n).astype(np.float32), 1.0))
+    out.append(("below", (rng.random(n) * np.float32(-1e-6)).astype(np.float32), 1.0))
+    out.append(("ramp", np.linspace(-110, 0, n).astype(np.float32), 1.0))
+    out.append(("fall", np.linspace(0, -110, n).astype(np.float32), 1.0))
+    late = spread.copy()
+    late[-1] = 40.0
+    out.append(("late", late, 1.0))
+    some = spread.copy()
+    some[rng.integers(0, n, n // 3)] = -np.inf
+    out.append(("-inf", some, 1.0))
+    nan = spread.copy()
+    nan[n // 2] = np.nan
+    out.append(("nan", nan, 1.0))
+    return out
+
+
+@pytest.mark.parametrize("n", [2047, 2048, 2049, 2055, 4097, 32768, 151936, 524288, 524289])
+def test_sampler_sum_bits(oracle, gpu, n):
+    """The sum itself, from the head of a draw's scratch, against numpy's
+    sequential float32 accumulate of the draw's own exponentials (samples of
+    them against the oracle's expf), bit for bit; both ways of taking it, the
+    composed runs and the one workgroup, occur where the runs apply."""
+    say("test_sampler_sum_bits n=%d" % n)
+    ds = DevSampler(gpu, n)
+    e_at = 256 + 256 * 8  # the state, the 256 partial maxima, then the exponentials
+    runs = 2048 <= n <= 524288
+    walked, alone = [], []
+    try:
+        for name, lg, t in _sum_cases(n):
+            ds.draws(lg, t, 0.9, 5, 1)
+            head = gpu.download(ds.d_scratch, (5,), np.int32)
+            e = gpu.download(ds.d_scratch + e_at, (n,), np.float32)
+            with np.errstate(invalid="ignore"):
+                x = ((lg - lg[head[0]]) / np.float32(t)).astype(np.float32)
+            for i in list(range(0, n, max(1, n // 200))) + [n - 1]:
+                want = np.float32(oracle.lib().orc_expf(float(x[i])))
+                assert e[i] == want or (np.isnan(e[i]) and np.isnan(want)), (name, i)
+            want = np.add.accumulate(e, dtype=np.float32)[-1:]
+            got = head[1:2].view(np.float32)
+            assert np.array_equal(got.view(np.uint32), want.view(np.uint32)) or \
+                (np.isnan(got[0]) and np.isnan(want[0])), (name, float(got[0]), float(want[0]))
+            (walked if head[2] >= 0 else alone).append(name)
+        say("  composed: %s; one workgroup: %s" % (" ".join(walked), " ".join(alone)))
+        if runs:
+            assert "equal" in walked and "nan" in alone
+            assert sum(w.startswith("model") for w in walked) >= 12
+        else:
+            assert not walked
+    finally:
+        ds.close()
+
+
 def _chain_cases():
     """Vectors for the running sums: (name, values, thresholds)."""
     rng = np.random.default_rng(31)
