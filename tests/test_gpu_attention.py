@@ -160,18 +160,19 @@ def test_batch_rows_on_matrix_cores(n):
             lay.close()
 
 
-def test_batch_in_passes():
+@pytest.mark.parametrize("n", [130, 131])
+def test_batch_in_passes(n):
     """A context whose score matrix takes two passes (67 tokens of it fit the
-    bounded scratch)."""
+    bounded scratch): of 65 tokens each, and of 66 and 65; every token."""
     torch = pytest.importorskip("torch")
-    say("test_batch_in_passes")
-    n, pos = 130, 60000
+    say("test_batch_in_passes n=%d" % n)
+    pos = 60000
     lay = Layer(torch, 256, 32, 4, pos + n, 5)
     try:
         kc, vc = lay.cache(pos)
         x = lay.up(lay.rng.standard_normal((n, 256)).astype(np.float32))
         got = lay.batch(x, kc, vc, pos)
-        for i in (0, 1, 66, 67, 68, 129):
+        for i in range(n):
             want = lay.token(x[i:i + 1], kc, vc, pos + i)
             assert np.array_equal(bits(got[i:i + 1]), bits(want)), "token %d" % i
     finally:

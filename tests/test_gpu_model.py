@@ -319,9 +319,9 @@ def test_model_prefill_equals_feeds_golden(oracle, tmp_path, name):
 def test_model_full_shape_prefill_equals_feeds(n):
     """48 layers at the Qwen3-30B-A3B shape: an n-token prompt through
     mia_gpu_model_prefill, then steps, gives the logits bits of n feeds and
-    the same steps. 70 tokens: one batch, its MoE on the vector kernels (560
-    assignments); 300: one batch on the matrix-core kernels (2400); 1100: two
-    batches of 550, each nine 64-token row chunks (the last partial)."""
+    the same steps. One batch each; 70 tokens: its MoE on the vector kernels
+    (560 assignments); 300 and 1100: on the matrix-core kernels (2400 and 8800),
+    the attention's scores in tiles."""
     say("test_model_full_shape_prefill_equals_feeds n=%d" % n)
     a = M.GpuModel(None, 1200, synth=(QWEN_FULL, 9))
     b = M.GpuModel(None, 1200, synth=(QWEN_FULL, 9))
@@ -341,8 +341,8 @@ def test_model_full_shape_prefill_equals_feeds(n):
 
 
 def test_model_full_shape_prefill_far_positions():
-    """A prompt batch whose context is too long for its scores in LDS (the
-    scores in device memory, 64 tokens per pass: 70 tokens at positions
+    """A prompt batch whose context is too long for its scores in LDS (in
+    tiles of a score matrix in device memory: 70 tokens at positions
     4300 .. 4369), against feeds; the positions before are left empty (zero
     cache rows) on both handles."""
     say("test_model_full_shape_prefill_far_positions")
@@ -366,6 +366,31 @@ def test_model_full_shape_prefill_far_positions():
         b.close()
 
 
+@pytest.mark.parametrize("n,pos", [(2047, 0), (2048, 0), (2049, 0), (2101, 5), (4500, 0)])
+def test_model_prefill_of_several_batches(n, pos):
+    """Prompts around and above the 2048 tokens of a batch (the largest batch,
+    two of equal size and of sizes one apart, three), the first positions
+    already there, against feeds: the logits bits of the steps after."""
+    say("test_model_prefill_of_several_batches n=%d pos=%d" % (n, pos))
+    cfg = dict(QWEN_FULL, n_layers=3, vocab=4000)
+    a = M.GpuModel(None, n + pos + 3, synth=(cfg, 19))
+    b = M.GpuModel(None, n + pos + 3, synth=(cfg, 19))
+    try:
+        toks = np.random.default_rng(n).integers(0, cfg["vocab"], pos + n + 3).tolist()
+        for p in range(pos):
+            a.feed(toks[p], p)
+        a.prefill(toks[pos:pos + n], pos)
+        for p in range(pos + n):
+            b.feed(toks[p], p)
+        for p in range(pos + n, pos + n + 3):
+            la, lb = a.step(toks[p], p), b.step(toks[p], p)
+            assert np.all(np.isfinite(la))
+            assert np.array_equal(bits(la), bits(lb)), "position %d" % p
+    finally:
+        a.close()
+        b.close()
+
+
 def test_model_stack_long_contexts():
     """Positions from which the model stack spreads a head over its XCD, on a
     context filled by a prompt: around the switch (position 33), the ends of
@@ -379,6 +404,7 @@ def test_model_stack_long_contexts():
     m = M.GpuModel(None, n, synth=(cfg, 17))
     try:
         rng = np.random.default_rng(15)
+        m.trace()  # (raises unless the stack runs at this shape and length)
         m.prefill(rng.integers(0, cfg["vocab"], n - 1).tolist(), 0)
         for p in (n - 1, 5375, 5119, 4096, 4095, 2560, 2559, 2047, 671, 672, 336, 335, 320, 319, 318,
                   224, 223, 113, 112, 111, 64, 35, 34, 33, 32, 31):
