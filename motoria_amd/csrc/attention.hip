@@ -983,8 +983,8 @@ int mhip_attention_batch(mhip_ctx *c, const mhip_attn_dims *s, const float *d_at
                    {q, k, v},
                    {0, qd, qd + kvd, qd + 2 * kvd}};
     // the matrix cores when the layer's weights are packed (a layer's call at
-    // position 0, us, vector rows / matrix cores: 2 tokens 83/74, 16 90/81,
-    // 100 131/94, 400 347/171, 1024 824/384)
+    // position 0, us, vector rows / matrix cores: 1 token 76/67, 2 83/74, 16
+    // 90/81, 100 131/94, 400 347/171, 1024 824/384)
     const bool mm = d_pack && mhip::rows_pack_fits(s);
     if (mm) {
         mhip::rows_token_frags(st, xq, xs, n, nb, ld, xh, xst);

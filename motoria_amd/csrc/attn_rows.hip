@@ -20,9 +20,14 @@
 // issues a vector operation at half the rate of several. Measured at 777 tokens (QKV 5120 x 2048, O 2048 x 4096): 51 us a
 // launch, against 145-160 us for operands in registers one block ahead
 // (about 17 us is what the products and their terms take).
+#include "attn_common.h"
 #include "mhip_internal.h"
 
 namespace {
+
+using mhip_attn::dma16;
+using mhip_attn::dma4;
+using mhip_attn::wait_vm;
 
 constexpr int QK = mhip::QK;
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
@@ -77,23 +82,6 @@ struct RowPack {
     float *out[3];
     int r0[4];             // rows of segment k: [r0[k], r0[k+1]), multiples of RM_R
 };
-
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-// global -> LDS, 16 (resp. 4) bytes per lane, lane i's at lds + 16 i (4 i);
-// lds wave-uniform, completion counted by vmcnt.
-__device__ __forceinline__ void dma16(unsigned lds, const void *g) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(g)
-                 : "memory", "m0");
-}
-__device__ __forceinline__ void dma4(unsigned lds, const void *g) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(g)
-                 : "memory", "m0");
-}
-#pragma clang diagnostic pop
-template <int N> __device__ __forceinline__ void wait_vm() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
 
 template <int NJ> struct alignas(16) Step {
     _Float16 w[RM_R / 16][FRAG];  // 4 KB

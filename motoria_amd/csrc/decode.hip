@@ -57,11 +57,11 @@
 // MHIP_DECODE_CERTIFIED from the parallel logits (relative error ~1e-6
 // against the reference's) unless the exact fallback ran for that layer.
 //
-// The same body (decode_body.inc) compiles twice: k_decode_stack, the MoE
-// alone, and k_model_stack, which runs each layer's attention (attn_stage:
-// rmsnorm, Q/K/V rows, the 32 heads with the KV cache, Wo and the residual,
-// src/model/forward.c:118-165) before that layer's MoE, so a whole decode
-// token is one launch (forward.c:210-213).
+// The same body (decode_body.inc) compiles three times: k_decode_stack, the
+// MoE alone, and k_model_stack and k_model_stack_long (by position), which run
+// each layer's attention (attn_stage: rmsnorm, Q/K/V rows, the 32 heads with
+// the KV cache, Wo and the residual, src/model/forward.c:118-165) before that
+// layer's MoE, so a whole decode token is one launch (forward.c:210-213).
 #include <cstring>
 #include <mutex>
 #include <type_traits>
@@ -1351,7 +1351,7 @@ __device__ __forceinline__ void attn_stage(const DecodeArgs &a, Lds &sh, DecodeW
     TRACE(31);
 }
 
-// The kernels: one body (decode_body.inc) compiled twice.
+// The kernels: one body (decode_body.inc) compiled three times.
 __global__ __launch_bounds__(NT) void k_decode_stack(DecodeArgs a) {
 #define DECODE_ATTN 0
 #include "decode_body.inc"

@@ -10,16 +10,16 @@
 // v_mfma_f32_16x16x32_f16 over one 32-value block gives the exact int32
 // block dot (every partial sum is an integer below 2^24). The reference's
 // block term ((float)acc * d_w) * d_x is added to the row sum in block order
-// by the vector ALUs (matmul.c:19-28). gate/up keeps the reference's three
-// roundings, so h, and Q8(h) after it, are bit-equal to the reference's: h
-// is requantized, and a code that flips on a last-ulp difference moves a
-// token's layer output by up to ~1.5e-3 relative (measured over 48 layers of
-// 4096 tokens with one fused multiply-add there). down, whose output is not
-// requantized, adds each term with one fused multiply-add (the second
-// product's rounding and the addition's become one): the expert outputs are
-// within a few fp32 ulps of the reference's. gate/up writes Q8(h) as fp16
-// codes plus block-major scales, which down reads the same way as gate/up
-// reads Q8(xn); no operand is ever rounded to fp16.
+// by the vector ALUs (matmul.c:19-28) with the reference's three roundings, so
+// h, Q8(h) after it and the expert outputs are bit-equal to the reference's.
+// In gate/up that is needed: h is requantized, and a code that flips on a
+// last-ulp difference moves a token's layer output by up to ~1.5e-3 relative
+// (measured over 48 layers of 4096 tokens with one fused multiply-add there).
+// down, whose output is not requantized, has the fused form as an option
+// (MHIP_FAST_DOWN: the second product's rounding and the addition's become
+// one, within a few fp32 ulps). gate/up writes Q8(h) as fp16 codes plus
+// block-major scales, which down reads the same way as gate/up reads Q8(xn);
+// no operand is ever rounded to fp16.
 //
 // Tiles: 256 weight rows x 128 assignments (rows of one expert's bucket),
 // one 32-value Q8_0 block of k per step, eight wavefronts and two workgroups
@@ -33,7 +33,7 @@
 // wavefront's (one alone issues one every ~4.3 cycles, several together one
 // every ~2.1). Against four wavefronts of 64 weight rows x 128 assignments
 // (two per SIMD), same-box: gate/up + down 151 + 80 -> 133 + 75 us at T =
-// 512; the layer 598 -> 572 at T = 2048 skewed, 914 -> 905 at T = 4096.
+// 512; the layer 598 -> 576 at T = 2048 skewed; T = 4096 the same (895, 898).
 //
 // Operands move from global memory straight into an NS-stage LDS ring with
 // global_load_lds (no registers on the way), NS-1 steps ahead of the
@@ -524,8 +524,8 @@ __global__ __launch_bounds__(GT, 4) void k_gateup_mfma(
 // blockIdx.x = tile of assignment rows x 8 column tiles of 256 consecutive
 // down rows n0..n0+255. The x operand is the tile's Q8(h) (fp16 codes,
 // bucketed order, contiguous) with its block-major scales. Results go out
-// through LDS a wavefront's 64 columns at a time, so every assignment row is
-// written as 256 contiguous bytes.
+// through LDS 128 columns at a time, so every assignment row is written as
+// 512 contiguous bytes.
 // EXACT: the reference's roundings of each block term (the expert outputs
 // bit-equal); otherwise one fused multiply-add per term (a few ulps).
 template <bool EXACT>
