@@ -46,6 +46,11 @@
 #include "mia/model_gpu.h"
 #include "mia/serve.h"
 
+/* PREFILL_CHUNK: the prompt tokens of one mia_gpu_model_prefill call, which is
+ * the step in which a cancel is noticed and PROG moves: 34 ms at the
+ * Qwen3-30B-A3B shape (81 for the 2048 tokens that the library takes as a
+ * batch). It costs reading the experts once more: 1400 tokens 59 ms so and 49
+ * in one call, 3000 tokens 155 and 149. */
 enum { MESSAGE_MAX = 1 << 20, PREFILL_CHUNK = 1024 };
 
 static volatile sig_atomic_t g_stop_turn;
