@@ -15,11 +15,12 @@
 // A workgroup takes 64 weight rows x 32 NJ tokens, a wavefront half of each
 // (2 x NJ tiles of 16 x 16), one block per step of an RS-stage LDS ring
 // filled RS - 1 steps ahead. What bounds it is the vector ALUs: twelve
-// operations per matrix instruction, and the matrix cores do not run beside
-// them; the small tiles buy four wavefronts per SIMD, and one wavefront alone
-// issues a vector operation at half the rate of several. Measured at 777 tokens (QKV 5120 x 2048, O 2048 x 4096): 51 us a
-// launch, against 145-160 us for operands in registers one block ahead
-// (about 17 us is what the products and their terms take).
+// operations per matrix instruction, beside which the matrix cores run for
+// about 40 % of their time; the small tiles buy four wavefronts per SIMD, and
+// one wavefront alone issues a vector operation at half the rate of several.
+// Measured at 777 tokens (QKV 5120 x 2048, O 2048 x 4096): 51 us a launch,
+// against 145-160 us for operands in registers one block ahead (about 17 us is
+// what the products and their terms take).
 #include "attn_common.h"
 #include "mhip_internal.h"
 
