@@ -56,8 +56,10 @@ int mia_gpu_model_feed(mia_gpu_model *m, int token, int pos);
  * through each layer at once (the attention of the batch with
  * mhip_attention_batch, its MoE on the per-stage kernels for T tokens, the
  * matrix-core ones from MHIP_GEMM_MIN_A assignments on), so the weights are
- * read once per batch instead of once per token. The KV rows written are bit-equal to n calls of
- * mia_gpu_model_feed; no logits are formed. 0 or -1. */
+ * read once per batch instead of once per token. The first call allocates the
+ * batch's buffers and packs the attention weights; without memory for them it
+ * fails and leaves nothing behind. The KV rows written are bit-equal to n calls
+ * of mia_gpu_model_feed; no logits are formed. 0 or -1. */
 int mia_gpu_model_prefill(mia_gpu_model *m, const int *tokens, int n, int pos);
 
 /* The token sampler (mhip_sample) on the logits of the last

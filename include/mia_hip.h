@@ -268,7 +268,8 @@ int mhip_decode_status(mhip_ctx *c, const void *d_ws, int status[4]);
  * through pinned memory (mhip_host_malloc): one small launch each, the second
  * with the call's one wait. mhip_decode_out leaves x [d], idx [nr], w [nr]
  * (32-bit words, in this order) and six words of its own at h_out, and the
- * launch's status as mhip_decode_status gives it. */
+ * launch's status as mhip_decode_status gives it. Null pointers are refused
+ * (d_idx and d_w only where nr > 0). */
 int mhip_decode_in(mhip_ctx *c, float *d_x, const float *h_x, int d);
 int mhip_decode_out(mhip_ctx *c, const void *d_ws, const float *d_x, int d, const int *d_idx,
                     const float *d_w, int nr, void *h_out, int status[4]);
@@ -312,7 +313,8 @@ int mhip_attention(mhip_ctx *c, const mhip_attn_dims *s, const float *d_attn_nor
  * are bit-equal to n calls of mhip_attention in position order (the rows of
  * all n tokens are appended before any score; token t reads rows
  * 0 .. pos + t). d_scratch: mhip_attention_batch_scratch_bytes(s, n,
- * max_seq) bytes (0 for invalid arguments). */
+ * max_seq) bytes (0 for invalid arguments). Null pointers other than d_pack
+ * are refused. */
 size_t mhip_attention_batch_scratch_bytes(const mhip_attn_dims *s, int n, int max_seq);
 int mhip_attention_batch(mhip_ctx *c, const mhip_attn_dims *s, const float *d_attn_norm,
                          const void *d_wq, const void *d_wk, const void *d_wv, const void *d_wo,
@@ -321,11 +323,11 @@ int mhip_attention_batch(mhip_ctx *c, const mhip_attn_dims *s, const float *d_at
                          const void *d_pack, void *d_scratch, int flags);
 /* The layer's Q, K, V and O weights repacked for mhip_attention_batch's
  * matrix-core rows (no counterpart in the reference): codes as fp16
- * integers in the matrix instruction's order, scales block-major; d_pack holds mhip_attention_pack_bytes(s)
- * bytes (0 for shapes whose rows are not multiples of 64, which keep the
- * vector kernels). With d_pack given, the batch's
- * Q/K/V and O rows form on the matrix cores, with the same bits (exact block
- * dots, block terms in block order); NULL keeps the vector kernels. */
+ * integers in the matrix instruction's order, scales block-major; d_pack holds
+ * mhip_attention_pack_bytes(s) bytes (0 for shapes whose rows are not multiples
+ * of 64, which keep the vector kernels). With d_pack given, the batch's Q/K/V
+ * and O rows form on the matrix cores, with the same bits (exact block dots,
+ * block terms in block order); NULL keeps the vector kernels. */
 size_t mhip_attention_pack_bytes(const mhip_attn_dims *s);
 int mhip_attention_pack(mhip_ctx *c, const mhip_attn_dims *s, const void *d_wq, const void *d_wk,
                         const void *d_wv, const void *d_wo, void *d_pack);

@@ -398,9 +398,10 @@ __global__ __launch_bounds__(SQ_T) void k_chain_sum(const float *__restrict__ e,
 // being of values >= 0, it did all along. Where that fails, or with more
 // than WALK_MAX noted pieces (NaN or infinite values, sums among the
 // subnormals), seq_scan runs over all values instead. 151936 values: 108 us
-// for seq_scan on one workgroup, 4 + 8 us for the two; about one in twenty
-// of a model's logits at T = 0.6-1 still needs seq_scan (many values too small
-// to be added move a power of two past its noted pieces).
+// for seq_scan on one workgroup, 4 + 8 us for the two; 3-8 % of draws over
+// model-like logits at T = 0.6-1 still need seq_scan (many values too small
+// to be added move a power of two past its noted pieces) and take what every
+// draw took on one workgroup.
 struct Run {
     int a0, a1;  // added to even (odd) bits
     int P;       // the exponent field of the binade; 0: nothing is added
